@@ -436,8 +436,8 @@ void VCycleMG::vcycle_mixed(const double *r) {
         });
     } else {
         d.timed("mg_tail", f, [&] {
-            mg_tail(s, m_plan_dev + 1, m_res1[f]->data, m_tail_lds_bytes[1], precond_coarse_iter(), m_mixed_tail,
-                    m_mixed_tail > 0 ? m_mixed_weight : 0.0, true, m_pc_tol);
+            mg_tail(s, m_plan_dev + 1, m_res1[f]->data, m_tail_lds_bytes[1], m_tail_box, precond_coarse_iter(),
+                    m_mixed_tail, m_mixed_tail > 0 ? m_mixed_weight : 0.0, true, m_pc_tol);
         });
     }
     for (int level = f; level > 0; --level) {
@@ -564,6 +564,8 @@ void VCycleMG::build_tail() {
         T.err0 = l < L ? m_err0[l]->data : nullptr;
         for (int a = 0; a < 5; a++) T.lds_off[a] = -1;
     }
+    m_tail_box = 0;
+    for (int l = f; l < L; l++) m_tail_box = std::max(m_tail_box, d.level(l).n[0] * d.level(l).n[1] * d.level(l).n[2]);
     // LDS placement, coarsest level first, whole levels, while they fit.
     // Plan 0 serves the reference's V-cycle; plan 1 the launches that skip
     // the coarsest level (skip_dead): there the coarsest level is never
@@ -925,10 +927,10 @@ void VCycleMG::vcycle_fused(Field &out, const Field &b) {
     } else if (f < L) {
         d.timed("mg_tail", f, [&] {
             if (m_precond_call)
-                mg_tail(d.stream(), m_plan_dev + 1, f == 0 ? b.data : m_res1[f]->data, m_tail_lds_bytes[1],
+                mg_tail(d.stream(), m_plan_dev + 1, f == 0 ? b.data : m_res1[f]->data, m_tail_lds_bytes[1], m_tail_box,
                         precond_coarse_iter(), 0, 0.0, true, m_pc_tol);
             else
-                mg_tail(d.stream(), m_plan_dev, f == 0 ? b.data : m_res1[f]->data, m_tail_lds_bytes[0]);
+                mg_tail(d.stream(), m_plan_dev, f == 0 ? b.data : m_res1[f]->data, m_tail_lds_bytes[0], m_tail_box);
         });
     }
     for (int level = f; level > 0; --level) {

@@ -132,6 +132,7 @@ class VCycleMG : public IPressure {
     int m_tail_first = 0;          // first level of the single-workgroup kernel; n_level: none
     TailPlan *m_plan_dev = nullptr;     // [0] the reference's V-cycle, [1] with the coarsest level skipped
     int m_tail_lds_bytes[2] = {0, 0};
+    int m_tail_box = 0;                 // largest inner box the tail relaxes on
     // FP32 level arrays of the mixed V-cycle (levels above the tail)
     std::vector<float *> m_err1f, m_tmpf, m_scrf, m_res0f, m_res1f;
     int m_mixed_pre = 0, m_mixed_post = 0;  // sweeps of the mixed V-cycle (0: the XML's)
