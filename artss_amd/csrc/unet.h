@@ -18,7 +18,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <string>
 #include <vector>
 
 #include "unet_kernels.h"
@@ -50,25 +49,38 @@ class UNet {
   private:
     struct Layer {
         int ci, co, level;
-        float *W = nullptr, *b = nullptr, *gW = nullptr, *gb = nullptr;
-        float *mW = nullptr, *vW = nullptr, *mb = nullptr, *vb = nullptr;
-        uint16_t *W_bf = nullptr, *Wt_bf = nullptr;  // [27][ci][co], [27][co][ci]
-        uint16_t *Wup_bf = nullptr;  // layers on an upsampled input: nn::weights_up_bf16's form
+        size_t w, b;  // offsets of W and b in the flat parameter vector
+        uint16_t *fwd = nullptr, *bwd = nullptr;  // nn::WeightJob's BF16 copies
     };
     void ensure(int X, int Y, int Z);
+    void ensure_backward();
+    void refresh_weights();
+    const float *W(int layer) const { return m_params + m_layers[static_cast<size_t>(layer)].w; }
+    const float *B(int layer) const { return m_params + m_layers[static_cast<size_t>(layer)].b; }
     // keep_pre: store the decoder's pre-activations, which only the backward
     // pass of gradients() reads
     void run_forward(const float *x, bool keep_pre);
+    void run_backward(const float *target);
     void free_buffers();
     hipStream_t m_s;
     std::vector<Layer> m_layers;
+    // FP32 parameters, their gradients (and the loss after them) and Adam's
+    // moments, each one array in parameter order
+    float *m_params = nullptr, *m_grads = nullptr, *m_m = nullptr, *m_v = nullptr;
+    float *m_grads_host = nullptr;  // pinned
     int m_X = 0, m_Y = 0, m_Z = 0;
     std::vector<void *> m_buffers;
-    // activations (BF16) and gradients (FP32) at the current size
+    // activations (BF16) at the current size
     uint16_t *h0, *e0, *p1, *e1, *p2, *e2, *p3, *e3, *c2, *d2, *c1, *d1, *c0, *d0;
-    float *y, *gy, *g0a, *g0b, *g0c, *g1a, *g1b, *g1c, *g2a, *g2b, *g2c, *g3a, *g3b;
+    float *y;
+    // backward pass (allocated by the first gradients() at a size): skip
+    // gradients and encoder data gradients per level (FP32), masked gradients
+    // (BF16), the sums' partial rows
+    bool m_backward = false;
+    float *gy, *gs[3], *gp[3], *gh;
+    uint16_t *gm[4];
+    float *m_part = nullptr;
     const float *m_x = nullptr;
-    float *m_loss = nullptr, *m_loss_host = nullptr;
     int m_adam_t = 0;
 };
 

@@ -2,19 +2,22 @@
 //
 // Tensors are channels-last (voxel-major, channel innermost) at the
 // resolution of their level, without ghost cells.  Activations and weights
-// are BF16 (raw bit patterns, round-to-nearest-even), gradients FP32, and
-// every product accumulates in FP32.  The 3x3x3 convolutions with 16 or more
-// channels on both sides are implicit GEMMs on the gfx950 matrix cores.
-// The forward pass (k_conv_fwd, the one the warm start runs every step) uses
-// v_mfma_f32_16x16x32_bf16 with a register tile per wavefront (see there);
-// the gradient kernels use v_mfma_f32_16x16x16_bf16: a wavefront owns 16
-// consecutive voxels along x and all output channels; per tap and 16-channel
-// chunk it loads one 16x16 BF16 operand of the input (8 bytes per lane,
-// contiguous in the channel) and one of the weights per output tile.
-// Operand layouts of the 16x16x16 form:
-//   A (16x16, rows m, cols k): lane l holds A[l%16][4*(l/16) .. +3]
-//   B (16x16, rows k, cols n): lane l holds B[4*(l/16) .. +3][l%16]
-//   D (16x16 FP32):            lane l holds D[4*(l/16) .. +3][l%16]
+// are BF16 (raw bit patterns, round-to-nearest-even), gradients FP32 (rounded
+// to BF16 as matrix operands), and every product accumulates in FP32.  The
+// 3x3x3 convolutions with 16 or more channels on both sides, forward and
+// backward, are implicit GEMMs on v_mfma_f32_16x16x32_bf16 with register
+// tiles per wavefront (k_conv_fwd, k_conv_up_dgrad, k_conv_wgrad); the weight
+// gradients of the two end layers, whose inputs are FP32 on one side, run on
+// v_mfma_f32_16x16x4_f32.  Operand layouts:
+//   16x16x32 BF16, A (rows m) and B (columns n): lane l holds row or column
+//     l%16 and eight k values; both operands give a lane's slot the same k,
+//     so their order does not change the sum
+//   16x16x4 FP32, A and B: lane l holds row or column l%16, k = l/16
+//   D (16x16 FP32): lane l holds D[4*(l/16) .. +3][l%16]
+//
+// Sums over voxels (weight and bias gradients, the loss) go to one partial
+// row per workgroup, and one launch adds the rows in a fixed order
+// (k_sum_rows): the gradients are the same bits in every run.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -37,7 +40,11 @@ __device__ inline uint16_t f2bf(float f) {
     u += 0x7FFFu + ((u >> 16) & 1u);  // round to nearest even (finite inputs)
     return static_cast<uint16_t>(u >> 16);
 }
-__device__ inline short f2bfs(float f) { return static_cast<short>(f2bf(f)); }
+// whether a BF16 bit pattern is > 0
+__device__ inline bool positive(unsigned b) { return __uint_as_float(b << 16) > 0.f; }
+__device__ inline unsigned pack2(float lo, float hi) {
+    return static_cast<unsigned>(f2bf(lo)) | (static_cast<unsigned>(f2bf(hi)) << 16);
+}
 
 __device__ inline long long vox(const Dims &D, int x, int y, int z) {
     return (static_cast<long long>(z) * D.Y + y) * D.X + x;
@@ -79,12 +86,20 @@ __device__ inline void tap_offset(int t, int &dx, int &dy, int &dz) {
 //   B (32x16): lane l holds column l%16, k = 8*(l/16) .. +7
 //   D (16x16 FP32): lane l holds D[4*(l/16) .. +3][l%16]
 // The epilogue stores the four channels a lane holds as one 8-byte write.
-template <int CIN, int COUT, bool UP, int NV>
+//
+// GRAD: the data gradient of a convolution that is not upsampled, the same
+// GEMM with mirrored taps: in is the output's gradient (BF16), CIN the
+// layer's output and COUT its input channels, Wt its weights as
+// [27][COUT][CIN] ([tap][c_in][c_out] of the layer), and gin receives FP32
+// sums, zero where the BF16 activation `skip` (optional) is not positive.
+template <int CIN, int COUT, bool UP, int NV, bool GRAD = false>
 __global__ void __launch_bounds__(256) k_conv_fwd(Dims D, const uint16_t *__restrict__ in,
                                                   const uint16_t *__restrict__ Wt, const float *__restrict__ bias,
                                                   uint16_t *__restrict__ out, uint16_t *__restrict__ pre,
-                                                  const uint16_t *__restrict__ skip, int relu) {
+                                                  const uint16_t *__restrict__ skip, int relu,
+                                                  float *__restrict__ gin) {
     static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channels come in tiles of 16");
+    static_assert(!(GRAD && UP), "k_conv_up_dgrad is the upsampling layers' data gradient");
     static_assert(!UP || (CIN >= 32 && NV % 2 == 0), "the upsampling form takes 32-channel K steps, tile pairs");
     constexpr int MT = COUT / 16;
     constexpr int KSTEPS = UP ? 8 * (CIN / 32) : (CIN >= 32 ? 27 * (CIN / 32) : 14);
@@ -144,6 +159,11 @@ __global__ void __launch_bounds__(256) k_conv_fwd(Dims D, const uint16_t *__rest
         const bool tap_ok = t < 27;
         int dx, dy, dz;
         tap_offset(tap_ok ? t : 0, dx, dy, dz);
+        if (GRAD) {
+            dx = -dx;
+            dy = -dy;
+            dz = -dz;
+        }
         bf16x8 a[MT], b[NV];
 #pragma unroll
         for (int ct = 0; ct < MT; ct++)
@@ -174,6 +194,18 @@ __global__ void __launch_bounds__(256) k_conv_fwd(Dims D, const uint16_t *__rest
 #pragma unroll
         for (int ct = 0; ct < MT; ct++) {
             const int co = ct * 16 + 4 * kg;
+            if (GRAD) {
+                float4 g{acc[ct][j][0], acc[ct][j][1], acc[ct][j][2], acc[ct][j][3]};
+                if (skip) {
+                    const uint2 m = *reinterpret_cast<const uint2 *>(skip + v * COUT + co);
+                    g.x = positive(m.x & 0xFFFFu) ? g.x : 0.f;
+                    g.y = positive(m.x >> 16) ? g.y : 0.f;
+                    g.z = positive(m.y & 0xFFFFu) ? g.z : 0.f;
+                    g.w = positive(m.y >> 16) ? g.w : 0.f;
+                }
+                *reinterpret_cast<float4 *>(gin + v * COUT + co) = g;
+                continue;
+            }
             float c4[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) c4[e] = acc[ct][j][e] + bias[co + e];
@@ -311,301 +343,589 @@ __global__ void k_down(Dims D, const uint16_t *__restrict__ in, uint16_t *__rest
 }
 
 // ---------------------------------------------------------------- backward
-// gin[v][ci] = sum_t sum_co gout[v - off_t][co] * W[t][ci][co] (zero outside);
-// W is [27][CIN][COUT]; gout FP32 (rounded to BF16 as the matrix operand).
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(256) k_conv_dgrad(Dims D, const float *__restrict__ gout,
-                                                    const uint16_t *__restrict__ W, float *__restrict__ gin) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int x0 = (blockIdx.x * 4 + wave) * 16;
-    const int y = blockIdx.y, z = blockIdx.z;
-    if (x0 >= D.X) return;
-    const int vx = x0 + (lane & 15), kq = lane >> 4;
-    f32x4 acc[CIN / 16];
-#pragma unroll
-    for (int ct = 0; ct < CIN / 16; ct++) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int t = 0; t < 27; t++) {
-        int dx, dy, dz;
-        tap_offset(t, dx, dy, dz);
-        const int xx = vx - dx, yy = y - dy, zz = z - dz;
-        const bool inside = vx < D.X && xx >= 0 && xx < D.X && yy >= 0 && yy < D.Y && zz >= 0 && zz < D.Z;
-        const long long src = inside ? vox(D, xx, yy, zz) : 0;
-#pragma unroll
-        for (int c0 = 0; c0 < COUT; c0 += 16) {
-            bf16x4 b = bf16x4{0, 0, 0, 0};
-            if (inside) {
-                const float *g = gout + src * COUT + c0 + 4 * kq;
-                b = bf16x4{f2bfs(g[0]), f2bfs(g[1]), f2bfs(g[2]), f2bfs(g[3])};
-            }
-#pragma unroll
-            for (int ct = 0; ct < CIN / 16; ct++) {
-                const bf16x4 a = *reinterpret_cast<const bf16x4 *>(
-                    W + (static_cast<long long>(t) * CIN + ct * 16 + (lane & 15)) * COUT + c0 + 4 * kq);
-                acc[ct] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[ct], 0, 0, 0);
-            }
-        }
-    }
-    if (vx >= D.X) return;
-    const long long v = vox(D, vx, y, z);
-#pragma unroll
-    for (int ct = 0; ct < CIN / 16; ct++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) gin[v * CIN + ct * 16 + 4 * kq + e] = acc[ct][e];
+// One 64-bit transposed LDS read per lane: with the 16 lanes of a group
+// pointing at four voxels (lane 4 i + q at channels 4 q .. 4 q + 3 of voxel
+// i), lane c of the group receives channel c of the four voxels.
+__device__ inline bf16x4 lds_transposed(const uint16_t *p) {
+    typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+    return __builtin_bit_cast(
+        bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4 *)(const_cast<uint16_t *>(p))));
+}
+__device__ inline bf16x8 join(bf16x4 a, bf16x4 b) {
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// gW[t][ci][co] += sum_v in[v + off_t][ci] * gout[v][co] over this
-// workgroup's x-lines (grid: line blocks x 27 taps).  Each wavefront
-// accumulates its lines' 16-voxel chunks as matrix products with the voxels
-// as the reduction index, then adds its tiles to gW with FP32 atomics.
-// UP: the forward read `in` nearest-upsampled from half resolution.
+// Weight gradient of a 3x3x3 convolution, partial sums:
+// part[block][t][ci][co] = sum over the block's voxels v of
+// in[v + off_t][ci] * g[v][co], both BF16, FP32 accumulation.
+//
+// A matrix product over the voxels: A is in^T (rows ci), B is g (columns co),
+// K = 32 voxels per instruction.  A workgroup covers the nine taps of one z
+// offset (blockIdx.y), one wavefront per y offset with the three x offsets in
+// its registers.  It stages rows of g and of `in` with a one-voxel halo in
+// LDS as they lie in memory, [voxel][channel] (zero outside the volume), and
+// reads operands with the transposing LDS read: a tap is only another base
+// address, and an operand of g serves three taps.  Voxels are padded to an
+// odd multiple of 32 bytes where they are 64 bytes or more, so that the eight
+// voxels a read touches at once lie in different banks.  UP: `in` lives at
+// half resolution; a fine voxel's operand address is that of its coarse voxel.
+//
+// With two-byte gathers from memory and one atomic per weight and wavefront
+// the layers of a 128x64x64 volume took 1400 us together; so they take 185 us.
+constexpr int kGradVoxels = 256;  // voxels per staged block (about), multiple of 32
+constexpr int kGradSegment = 128; // longest x segment of a block
+template <int C>
+constexpr int lds_voxel() {
+    return C == 16 ? 16 : C + 16;  // uint16 per voxel
+}
+struct GradBlocks {
+    int xb, rows;        // voxels along x and rows along y of a block
+    int nx, ny, blocks;  // blocks along x and y, in all
+};
+inline GradBlocks grad_blocks(Dims D) {
+    GradBlocks b;
+    b.xb = D.X < kGradSegment ? D.X : kGradSegment;
+    int rows = kGradVoxels / b.xb;
+    rows = rows < 2 ? 2 : (rows > 64 ? 64 : rows & ~1);
+    const int even = (D.Y + 1) & ~1;
+    b.rows = rows < even ? rows : even;
+    b.nx = (D.X + b.xb - 1) / b.xb;
+    b.ny = (D.Y + b.rows - 1) / b.rows;
+    b.blocks = b.nx * b.ny * D.Z;
+    return b;
+}
 template <int CIN, int COUT, bool UP>
-__global__ void __launch_bounds__(256) k_conv_wgrad(Dims D, const uint16_t *__restrict__ in,
-                                                    const float *__restrict__ gout, float *__restrict__ gW,
-                                                    int lines_per_block) {
+__global__ void __launch_bounds__(192) k_conv_wgrad(Dims D, GradBlocks B, const uint16_t *__restrict__ in,
+                                                    const uint16_t *__restrict__ g, float *__restrict__ part) {
+    constexpr int GS = lds_voxel<COUT>(), IS = lds_voxel<CIN>(), MT = CIN / 16, NT = COUT / 16;
+    extern __shared__ __align__(16) uint16_t lds[];
+    const int fmax = (B.rows * B.xb + 31) & ~31;
+    const int rows_in = UP ? B.rows / 2 + 2 : B.rows + 2, xh = UP ? (B.xb + 1) / 2 + 2 : B.xb + 2;
+    uint16_t *sg = lds, *si = sg + fmax * GS;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int t = blockIdx.y;
-    int dx, dy, dz;
-    tap_offset(t, dx, dy, dz);
-    const int kq = lane >> 4, m = lane & 15;
-    f32x4 acc[COUT / 16][CIN / 16];
+    const int dz = static_cast<int>(blockIdx.y) - 1, dy = wave - 1;
+    const Dims C{UP ? D.X >> 1 : D.X, UP ? D.Y >> 1 : D.Y, UP ? D.Z >> 1 : D.Z};
+    f32x4 acc[3][MT][NT];
 #pragma unroll
-    for (int a = 0; a < COUT / 16; a++)
+    for (int d = 0; d < 3; d++)
 #pragma unroll
-        for (int b = 0; b < CIN / 16; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int lines = D.Y * D.Z;
-    const int chunks = (D.X + 15) / 16;
-    const int first = blockIdx.x * lines_per_block;
-    const int last = min(lines, first + lines_per_block);
-    for (int line = first + wave; line < last; line += 4) {
-        const int y = line % D.Y, z = line / D.Y;
-        for (int ch = 0; ch < chunks; ch++) {
-            // reduction index k = voxel 4*kq + e of this chunk
-            bf16x4 ga[COUT / 16], ib[CIN / 16];
+        for (int a = 0; a < MT; a++)
 #pragma unroll
-            for (int a = 0; a < COUT / 16; a++) ga[a] = bf16x4{0, 0, 0, 0};
+            for (int b = 0; b < NT; b++) acc[d][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the voxels (of 32 in a K step) whose chunk this lane's two reads fetch
+    const int k0 = 4 * (lane >> 4) + ((lane & 15) >> 2), q4 = 4 * (lane & 3);
+    for (int blk = blockIdx.x; blk < B.blocks; blk += gridDim.x) {
+        const int bx = blk % B.nx, by = (blk / B.nx) % B.ny, z = blk / (B.nx * B.ny);
+        if (z + dz < 0 || z + dz >= D.Z) continue;  // uniform over the workgroup
+        const int x0 = bx * B.xb, y0 = by * B.rows, zi = UP ? (z + dz) >> 1 : z + dz;
+        const int cx0 = UP ? (x0 >> 1) - 1 : x0 - 1, cy0 = UP ? (y0 >> 1) - 1 : y0 - 1;
+        for (unsigned q = threadIdx.x; q < static_cast<unsigned>(fmax * (COUT / 8)); q += 192) {
+            const unsigned f = q / (COUT / 8), c = q % (COUT / 8) * 8, r = f / B.xb;
+            const int x = x0 + static_cast<int>(f - r * B.xb), y = y0 + static_cast<int>(r);
+            uint4 v{0u, 0u, 0u, 0u};
+            if (static_cast<int>(r) < B.rows && x < D.X && y < D.Y)
+                v = *reinterpret_cast<const uint4 *>(g + vox(D, x, y, z) * COUT + c);
+            *reinterpret_cast<uint4 *>(sg + f * GS + c) = v;
+        }
+        for (unsigned q = threadIdx.x; q < static_cast<unsigned>(rows_in * xh * (CIN / 8)); q += 192) {
+            const unsigned p = q / (CIN / 8), c = q % (CIN / 8) * 8, r = p / xh;
+            const int x = cx0 + static_cast<int>(p - r * xh), y = cy0 + static_cast<int>(r);
+            uint4 v{0u, 0u, 0u, 0u};
+            if (x >= 0 && x < C.X && y >= 0 && y < C.Y)
+                v = *reinterpret_cast<const uint4 *>(in + vox(C, x, y, zi) * CIN + c);
+            *reinterpret_cast<uint4 *>(si + p * IS + c) = v;
+        }
+        __syncthreads();
+        for (int f0 = 0; f0 < fmax; f0 += 32) {
+            bf16x4 gb[2][NT], ia[2][3][MT];
 #pragma unroll
-            for (int b = 0; b < CIN / 16; b++) ib[b] = bf16x4{0, 0, 0, 0};
+            for (int h = 0; h < 2; h++) {
+                const int f = f0 + k0 + 16 * h;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int x = ch * 16 + 4 * kq + e;
-                if (x >= D.X) continue;
-                const long long v = vox(D, x, y, z);
+                for (int b = 0; b < NT; b++) gb[h][b] = lds_transposed(sg + f * GS + b * 16 + q4);
+                // positions past the block's last row (g is zero there) read the last row
+                const int r0 = f / B.xb, x = f - r0 * B.xb, r = r0 < B.rows ? r0 : B.rows - 1;
 #pragma unroll
-                for (int a = 0; a < COUT / 16; a++) ga[a][e] = f2bfs(gout[v * COUT + a * 16 + m]);
-                const int xx = x + dx, yy = y + dy, zz = z + dz;
-                if (xx < 0 || xx >= D.X || yy < 0 || yy >= D.Y || zz < 0 || zz >= D.Z) continue;
-                long long s;
-                if (UP) {
-                    const Dims C{D.X >> 1, D.Y >> 1, D.Z >> 1};
-                    s = vox(C, xx >> 1, yy >> 1, zz >> 1);
-                } else {
-                    s = vox(D, xx, yy, zz);
+                for (int d = 0; d < 3; d++) {
+                    const int px = UP ? ((x0 + x + d - 1) >> 1) - cx0 : x + d,
+                              py = UP ? ((y0 + r + dy) >> 1) - cy0 : r + dy + 1;
+#pragma unroll
+                    for (int a = 0; a < MT; a++) ia[h][d][a] = lds_transposed(si + (py * xh + px) * IS + a * 16 + q4);
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+#pragma unroll
+                for (int a = 0; a < MT; a++)
+#pragma unroll
+                    for (int b = 0; b < NT; b++)
+                        acc[d][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            join(ia[0][d][a], ia[1][d][a]), join(gb[0][b], gb[1][b]), acc[d][a][b], 0, 0, 0);
+        }
+        __syncthreads();
+    }
+    float *row = part + static_cast<size_t>(blockIdx.x) * (27 * CIN * COUT);
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int a = 0; a < MT; a++)
+#pragma unroll
+            for (int b = 0; b < NT; b++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int t = (dz + 1) * 9 + (dy + 1) * 3 + d, ci = a * 16 + 4 * (lane >> 4) + e,
+                              co = b * 16 + (lane & 15);
+                    row[(t * CIN + ci) * COUT + co] = acc[d][a][b][e];
+                }
+}
+
+// the workgroup's sum of one float4 per thread over the threads with the same
+// threadIdx.x % groups (a power of two up to 16), written by the first
+// `groups` threads to row[4 * group ..]; 256 threads
+__device__ inline void group_sums(float4 v, int groups, float *row) {
+    __shared__ float4 s[256];
+    s[threadIdx.x] = v;
+    __syncthreads();
+    for (int n = 128; n >= groups; n >>= 1) {
+        if (static_cast<int>(threadIdx.x) < n) {
+            const float4 a = s[threadIdx.x], b = s[threadIdx.x + n];
+            s[threadIdx.x] = float4{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w};
+        }
+        __syncthreads();
+    }
+    if (static_cast<int>(threadIdx.x) < groups) *reinterpret_cast<float4 *>(row + 4 * threadIdx.x) = s[threadIdx.x];
+}
+
+// Data gradient of an upsampling layer with the sum over the eight fine
+// children of a coarse voxel: gc[c][ci] = sum over the 4x4x4 fine voxels
+// 2 c - 1 .. 2 c + 2 of g[v][co] Wd[tap][ci][co], the transpose of the
+// 2x2x2-per-parity form k_conv_fwd evaluates forward.  64 taps instead of the
+// 27 x 8 of a fine-resolution gradient followed by the sum, and that fine
+// FP32 gradient (67 MB at 128x64x64) is never written.  A weight Wd is a sum
+// of up to eight BF16 weights, held as three BF16 terms (the rounded sum and
+// twice the rounded remainder: 24 bits), so that the products are those of
+// the 27-tap form and no weight is rounded twice.
+//
+// The workgroup's WAVES wavefronts share one tile of NV x 16 coarse voxels of
+// a row and split the 64 taps; their sums meet in LDS in a fixed order, and the epilogue writes the skip gradient (FP32, optional) and
+// the gradient under the mask act > 0 (BF16, the next products' operand), and
+// keeps the masked values' channel sums (the bias gradient) per workgroup.
+// Small levels have few row tiles: there blockIdx.y splits the input channels
+// as well, MT tiles of 16 per workgroup (d2's level of a 128x64x64 volume, 64
+// row tiles: 49 us with all four channel tiles in one workgroup, 17 us split).
+template <int CO, int CI, int NV, int WAVES, int MT>
+__global__ void __launch_bounds__(64 * WAVES) k_conv_up_dgrad(Dims D, const uint16_t *__restrict__ g,
+                                                       const uint16_t *__restrict__ Wd,
+                                                       const uint16_t *__restrict__ act, float *__restrict__ gskip,
+                                                       uint16_t *__restrict__ gmask, float *__restrict__ part) {
+    constexpr int TILES = MT * NV, TAPS = 64 / WAVES, STEPS = CO == 16 ? TAPS / 2 : TAPS * (CO / 32);
+    static_assert(TAPS >= 4 && TAPS <= 16, "a wavefront's taps lie in one z plane, whole rows of four");
+    __shared__ f32x4 sum[WAVES][TILES][64];
+    __shared__ float bias[WAVES][16 * MT];
+    const int ci0 = static_cast<int>(blockIdx.y) * (16 * MT);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kg = lane >> 4;
+    const Dims F{2 * D.X, 2 * D.Y, 2 * D.Z};
+    const int nx = (D.X + 16 * NV - 1) / (16 * NV), tiles = nx * D.Y * D.Z;
+
+    const bf16x8 zero8 = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
+    float4 bct[MT];
+#pragma unroll
+    for (int ct = 0; ct < MT; ct++) bct[ct] = float4{0.f, 0.f, 0.f, 0.f};
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int x0 = tile % nx * (16 * NV), y = (tile / nx) % D.Y, z = tile / (nx * D.Y);
+        f32x4 acc[MT][NV];
+#pragma unroll
+        for (int ct = 0; ct < MT; ct++)
+#pragma unroll
+            for (int j = 0; j < NV; j++) acc[ct][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int fz = 2 * z - 1 + wave * TAPS / 16;
+        if (fz >= 0 && fz < F.Z) {
+#pragma unroll 2
+            for (int st = 0; st < STEPS; st++) {
+                // tap jx + 4 jy + 16 jz and first channel of the lane's eight k values
+                const int t = wave * TAPS + (CO == 16 ? 2 * st + (kg >> 1) : st / (CO / 32));
+                const int c = CO == 16 ? 8 * (kg & 1) : st % (CO / 32) * 32 + 8 * kg;
+                const int fy = 2 * y - 1 + ((t >> 2) & 3);
+                const bool row_ok = fy >= 0 && fy < F.Y;
+                bf16x8 a[3][MT], b[NV];
+#pragma unroll
+                for (int h = 0; h < 3; h++)
+#pragma unroll
+                    for (int ct = 0; ct < MT; ct++)
+                        a[h][ct] = __builtin_bit_cast(
+                            bf16x8, *reinterpret_cast<const uint4 *>(
+                                        Wd + ((64 * h + t) * CI + ci0 + ct * 16 + col) * CO + c));
+#pragma unroll
+                for (int j = 0; j < NV; j++) {
+                    const int fx = 2 * (x0 + 16 * j + col) - 1 + (t & 3);
+                    b[j] = zero8;
+                    if (row_ok && fx >= 0 && fx < F.X)
+                        b[j] = __builtin_bit_cast(bf16x8,
+                                                  *reinterpret_cast<const uint4 *>(g + vox(F, fx, fy, fz) * CO + c));
                 }
 #pragma unroll
-                for (int b = 0; b < CIN / 16; b++) ib[b][e] = static_cast<short>(in[s * CIN + b * 16 + m]);
+                for (int h = 0; h < 3; h++)
+#pragma unroll
+                    for (int ct = 0; ct < MT; ct++)
+#pragma unroll
+                        for (int j = 0; j < NV; j++)
+                            acc[ct][j] =
+                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][ct], b[j], acc[ct][j], 0, 0, 0);
             }
-#pragma unroll
-            for (int a = 0; a < COUT / 16; a++)
-#pragma unroll
-                for (int b = 0; b < CIN / 16; b++)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ga[a], ib[b], acc[a][b], 0, 0, 0);
-        }
-    }
-    // D[m = co][n = ci]: lane holds co = a*16 + 4*kq + e, ci = b*16 + m
-#pragma unroll
-    for (int a = 0; a < COUT / 16; a++)
-#pragma unroll
-        for (int b = 0; b < CIN / 16; b++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int co = a * 16 + 4 * kq + e, ci = b * 16 + m;
-                atomicAdd(&gW[(static_cast<long long>(t) * CIN + ci) * COUT + co], acc[a][b][e]);
-            }
-}
-
-// weight gradients of the first layer (CI FP32 inputs -> CO outputs):
-// one thread per weight entry (t, ci, co) sums x[v + off_t][ci] * g[v][co]
-// over this workgroup's voxel range, then adds it to gW atomically.
-template <int CI, int CO>
-__global__ void k_conv_in_wgrad(Dims D, const float *__restrict__ x, const float *__restrict__ g,
-                                float *__restrict__ gW, long long voxels_per_block) {
-    const int q = threadIdx.x;
-    if (q >= 27 * CI * CO) return;
-    const int t = q / (CI * CO), ci = (q / CO) % CI, co = q % CO;
-    int dx, dy, dz;
-    tap_offset(t, dx, dy, dz);
-    const long long n = static_cast<long long>(D.X) * D.Y * D.Z;
-    const long long v0 = blockIdx.x * voxels_per_block, v1 = min(n, v0 + voxels_per_block);
-    float acc = 0.f;
-    for (long long v = v0; v < v1; v++) {
-        const int i = static_cast<int>(v % D.X), y = static_cast<int>((v / D.X) % D.Y),
-                  z = static_cast<int>(v / (static_cast<long long>(D.X) * D.Y));
-        const int xx = i + dx, yy = y + dy, zz = z + dz;
-        if (xx < 0 || xx >= D.X || yy < 0 || yy >= D.Y || zz < 0 || zz >= D.Z) continue;
-        acc += x[vox(D, xx, yy, zz) * CI + ci] * g[v * CO + co];
-    }
-    atomicAdd(&gW[q], acc);
-}
-
-// gradients of the last layer (CI BF16 inputs -> 1 FP32 output, no activation):
-// weights as above, one thread per (t, ci); d in by a separate pass
-template <int CI>
-__global__ void k_conv_out_wgrad(Dims D, const uint16_t *__restrict__ in, const float *__restrict__ gy,
-                                 float *__restrict__ gW, long long voxels_per_block) {
-    const int q = threadIdx.x;
-    if (q >= 27 * CI) return;
-    const int t = q / CI, ci = q % CI;
-    int dx, dy, dz;
-    tap_offset(t, dx, dy, dz);
-    const long long n = static_cast<long long>(D.X) * D.Y * D.Z;
-    const long long v0 = blockIdx.x * voxels_per_block, v1 = min(n, v0 + voxels_per_block);
-    float acc = 0.f;
-    for (long long v = v0; v < v1; v++) {
-        const int i = static_cast<int>(v % D.X), y = static_cast<int>((v / D.X) % D.Y),
-                  z = static_cast<int>(v / (static_cast<long long>(D.X) * D.Y));
-        const int xx = i + dx, yy = y + dy, zz = z + dz;
-        if (xx < 0 || xx >= D.X || yy < 0 || yy >= D.Y || zz < 0 || zz >= D.Z) continue;
-        acc += bf2f(in[vox(D, xx, yy, zz) * CI + ci]) * gy[v];
-    }
-    atomicAdd(&gW[q], acc);
-}
-template <int CI>
-__global__ void k_conv_out_dgrad(Dims D, const float *__restrict__ W, const float *__restrict__ gy,
-                                 float *__restrict__ gin) {
-    const long long n = static_cast<long long>(D.X) * D.Y * D.Z;
-    for (long long v = blockIdx.x * 256LL + threadIdx.x; v < n; v += 256LL * gridDim.x) {
-        const int i = static_cast<int>(v % D.X), y = static_cast<int>((v / D.X) % D.Y),
-                  z = static_cast<int>(v / (static_cast<long long>(D.X) * D.Y));
-        float acc[CI];
-#pragma unroll
-        for (int ci = 0; ci < CI; ci++) acc[ci] = 0.f;
-        for (int t = 0; t < 27; t++) {
-            int dx, dy, dz;
-            tap_offset(t, dx, dy, dz);
-            const int xx = i - dx, yy = y - dy, zz = z - dz;
-            if (xx < 0 || xx >= D.X || yy < 0 || yy >= D.Y || zz < 0 || zz >= D.Z) continue;
-            const float gs = gy[vox(D, xx, yy, zz)];
-#pragma unroll
-            for (int ci = 0; ci < CI; ci++) acc[ci] += gs * W[t * CI + ci];
         }
 #pragma unroll
-        for (int ci = 0; ci < CI; ci++) gin[v * CI + ci] = acc[ci];
+        for (int ct = 0; ct < MT; ct++)
+#pragma unroll
+            for (int j = 0; j < NV; j++) sum[wave][ct * NV + j][lane] = acc[ct][j];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < TILES; q += WAVES) {
+            const int w = q + wave;
+            if (w >= TILES) continue;
+            const int ct = w / NV, j = w % NV, vx = x0 + 16 * j + col, ci = ci0 + ct * 16 + 4 * kg;
+            if (vx >= D.X) continue;
+            f32x4 v = sum[0][w][lane];
+#pragma unroll
+            for (int p = 1; p < WAVES; p++) v += sum[p][w][lane];
+            const long long at = vox(D, vx, y, z) * CI + ci;
+            if (gskip) *reinterpret_cast<float4 *>(gskip + at) = float4{v[0], v[1], v[2], v[3]};
+            const uint2 m = *reinterpret_cast<const uint2 *>(act + at);
+            float4 k;
+            k.x = positive(m.x & 0xFFFFu) ? v[0] : 0.f;
+            k.y = positive(m.x >> 16) ? v[1] : 0.f;
+            k.z = positive(m.y & 0xFFFFu) ? v[2] : 0.f;
+            k.w = positive(m.y >> 16) ? v[3] : 0.f;
+            *reinterpret_cast<uint2 *>(gmask + at) = uint2{pack2(k.x, k.y), pack2(k.z, k.w)};
+#pragma unroll
+            for (int c2 = 0; c2 < MT; c2++)
+                if (c2 == ct) {
+                    bct[c2].x += k.x;
+                    bct[c2].y += k.y;
+                    bct[c2].z += k.z;
+                    bct[c2].w += k.w;
+                }
+        }
+        __syncthreads();
     }
-}
-
-// bias gradient: gb[c] += sum over voxels of g[v][c]
-template <int C>
-__global__ void k_bias_grad(long long n, const float *__restrict__ g, float *__restrict__ gb) {
-    __shared__ float part[C];
-    for (int q = threadIdx.x; q < C; q += blockDim.x) part[q] = 0.f;
+    // channel sums: over the 16 columns of a lane group, then the wavefronts
+#pragma unroll
+    for (int ct = 0; ct < MT; ct++) {
+        float v[4] = {bct[ct].x, bct[ct].y, bct[ct].z, bct[ct].w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            for (int off = 8; off > 0; off >>= 1) v[e] += __shfl_down(v[e], off, 16);
+            if (col == 0) bias[wave][ct * 16 + 4 * kg + e] = v[e];
+        }
+    }
     __syncthreads();
-    float acc[C];
+    if (static_cast<int>(threadIdx.x) < 16 * MT) {
+        float v = bias[0][threadIdx.x];
+        for (int p = 1; p < WAVES; p++) v += bias[p][threadIdx.x];
+        part[static_cast<size_t>(blockIdx.x) * CI + ci0 + threadIdx.x] = v;
+    }
+}
+
+// Gradient at an encoder layer's output: the skip gradient plus the spread
+// mean of the coarser level's (gc, at half resolution), under the mask act >
+// 0; BF16 operand of the next products and per-workgroup channel sums.
+template <int C>
+__global__ void __launch_bounds__(256) k_enc_grad(Dims D, const float *__restrict__ gskip,
+                                                  const float *__restrict__ gc, const uint16_t *__restrict__ act,
+                                                  uint16_t *__restrict__ gmask, float *__restrict__ part) {
+    constexpr int G = C / 4;
+    const Dims H{D.X >> 1, D.Y >> 1, D.Z >> 1};
+    const long long n = static_cast<long long>(D.X) * D.Y * D.Z * G;
+    float4 sum{0.f, 0.f, 0.f, 0.f};
+    for (long long q = blockIdx.x * 256LL + threadIdx.x; q < n; q += 256LL * gridDim.x) {
+        const unsigned v = static_cast<unsigned>(q / G);
+        const int c = static_cast<int>(q % G) * 4;
+        const unsigned r = v / static_cast<unsigned>(D.X);
+        const int x = static_cast<int>(v - r * D.X), y = static_cast<int>(r % D.Y), z = static_cast<int>(r / D.Y);
+        const float4 s = *reinterpret_cast<const float4 *>(gskip + q * 4);
+        const float4 p = *reinterpret_cast<const float4 *>(gc + vox(H, x >> 1, y >> 1, z >> 1) * C + c);
+        const uint2 m = *reinterpret_cast<const uint2 *>(act + q * 4);
+        float4 k;
+        k.x = positive(m.x & 0xFFFFu) ? s.x + 0.125f * p.x : 0.f;
+        k.y = positive(m.x >> 16) ? s.y + 0.125f * p.y : 0.f;
+        k.z = positive(m.y & 0xFFFFu) ? s.z + 0.125f * p.z : 0.f;
+        k.w = positive(m.y >> 16) ? s.w + 0.125f * p.w : 0.f;
+        *reinterpret_cast<uint2 *>(gmask + q * 4) = uint2{pack2(k.x, k.y), pack2(k.z, k.w)};
+        sum.x += k.x;
+        sum.y += k.y;
+        sum.z += k.z;
+        sum.w += k.w;
+    }
+    group_sums(sum, G, part + static_cast<size_t>(blockIdx.x) * C);
+}
+
+// Weight gradients of the end layers on the FP32 matrix instruction, four
+// voxels per instruction.  A wavefront takes whole x rows; lane l supplies
+// voxel l/16 of the four.  NM: row tiles of 16 of the product.
+template <int NM>
+__device__ inline void store_end_wgrad(f32x4 (&acc)[NM], int rows, float *row) {
+    __shared__ f32x4 s[4][NM][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-    for (int c = 0; c < C; c++) acc[c] = 0.f;
-    for (long long v = blockIdx.x * 256LL + threadIdx.x; v < n; v += 256LL * gridDim.x)
-#pragma unroll
-        for (int c = 0; c < C; c++) acc[c] += g[v * C + c];
-#pragma unroll
-    for (int c = 0; c < C; c++) atomicAdd(&part[c], acc[c]);
+    for (int a = 0; a < NM; a++) s[wave][a][lane] = acc[a];
     __syncthreads();
-    for (int q = threadIdx.x; q < C; q += blockDim.x) atomicAdd(&gb[q], part[q]);
-}
-
-// g *= (act > 0): the ReLU mask from stored BF16 activations
-__global__ void k_relu_mask(long long n, float *__restrict__ g, const uint16_t *__restrict__ act) {
-    for (long long q = blockIdx.x * 256LL + threadIdx.x; q < n; q += 256LL * gridDim.x)
-        if (!(bf2f(act[q]) > 0.f)) g[q] = 0.f;
-}
-
-// dst = src (the skip gradient) ; dst += src
-__global__ void k_copy_f(long long n, float *__restrict__ dst, const float *__restrict__ src) {
-    for (long long q = blockIdx.x * 256LL + threadIdx.x; q < n; q += 256LL * gridDim.x) dst[q] = src[q];
-}
-
-// coarse gradient of the 2x2x2 mean: gc (coarse dims D) spread /8 onto gf (fine) and added
-template <int C>
-__global__ void k_down_backward_add(Dims D, const float *__restrict__ gc, float *__restrict__ gf) {
-    const Dims F{D.X * 2, D.Y * 2, D.Z * 2};
-    const long long n = static_cast<long long>(F.X) * F.Y * F.Z * C;
-    for (long long q = blockIdx.x * 256LL + threadIdx.x; q < n; q += 256LL * gridDim.x) {
-        const int c = static_cast<int>(q % C);
-        const long long v = q / C;
-        const int x = static_cast<int>(v % F.X), y = static_cast<int>((v / F.X) % F.Y),
-                  z = static_cast<int>(v / (static_cast<long long>(F.X) * F.Y));
-        gf[q] += 0.125f * gc[vox(D, x >> 1, y >> 1, z >> 1) * C + c];
+    for (int a = wave; a < NM; a += 4) {
+        f32x4 v = s[0][a][lane];
+        for (int p = 1; p < 4; p++) v += s[p][a][lane];
+        for (int e = 0; e < 4; e++) {
+            const int m = a * 16 + 4 * (lane >> 4) + e;
+            if (m < rows) row[m * 16 + (lane & 15)] = v[e];
+        }
     }
 }
-
-// gradient of nearest upsampling: gc[v][c] = sum of the 8 fine children (D: coarse dims)
-template <int C>
-__global__ void k_up_backward(Dims D, const float *__restrict__ gf, float *__restrict__ gc) {
-    const Dims F{D.X * 2, D.Y * 2, D.Z * 2};
-    const long long n = static_cast<long long>(D.X) * D.Y * D.Z * C;
-    for (long long q = blockIdx.x * 256LL + threadIdx.x; q < n; q += 256LL * gridDim.x) {
-        const int c = static_cast<int>(q % C);
-        const long long v = q / C;
-        const int x = static_cast<int>(v % D.X), y = static_cast<int>((v / D.X) % D.Y),
-                  z = static_cast<int>(v / (static_cast<long long>(D.X) * D.Y));
-        float s = 0.f;
-        for (int o = 0; o < 8; o++) s += gf[vox(F, 2 * x + (o & 1), 2 * y + ((o >> 1) & 1), 2 * z + (o >> 2)) * C + c];
-        gc[q] = s;
+// first layer: rows m = 2 t + ci of x[v + off_t][ci], row 54 ones (the bias
+// gradient), columns co of g[v][co].  Thread-per-weight loops over the voxels
+// took 1331 us at 128x64x64 (a serial chain of 2048 voxels per thread);
+// 46 us so.
+constexpr int kInRows = 55;  // 27 taps x 2 channels and the bias
+__global__ void __launch_bounds__(256) k_conv_in_wgrad(Dims D, const float *__restrict__ x,
+                                                       const float *__restrict__ g, float *__restrict__ part) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m0 = lane & 15, k = lane >> 4;
+    f32x4 acc[4];
+    int dx[4], dy[4], dz[4];
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+        acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+        tap_offset((a * 16 + m0) / 2 < 27 ? (a * 16 + m0) / 2 : 13, dx[a], dy[a], dz[a]);
     }
+    const int lines = D.Y * D.Z;
+    for (int line = blockIdx.x * 4 + wave; line < lines; line += 4 * static_cast<int>(gridDim.x)) {
+        const int y = line % D.Y, z = line / D.Y;
+        const float *src[4];
+        bool ok[4];
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            const int yy = y + dy[a], zz = z + dz[a];
+            ok[a] = a * 16 + m0 < 54 && yy >= 0 && yy < D.Y && zz >= 0 && zz < D.Z;
+            src[a] = x + (ok[a] ? vox(D, 0, yy, zz) : 0) * 2 + (m0 & 1);
+        }
+        const float *gr = g + vox(D, 0, y, z) * 16;
+        for (int i = 0; i < D.X; i += 8) {  // sides are multiples of 8
+            float b[2], v[2][4];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                b[h] = gr[(i + 4 * h + k) * 16 + m0];
+#pragma unroll
+                for (int a = 0; a < 4; a++) {
+                    const int xx = i + 4 * h + k + dx[a];
+                    const bool in = ok[a] && xx >= 0 && xx < D.X;
+                    v[h][a] = src[a][in ? 2 * xx : 0];
+                    v[h][a] = in ? v[h][a] : 0.f;
+                }
+                v[h][3] = m0 == 6 ? 1.f : v[h][3];  // row 54
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int a = 0; a < 4; a++)
+                    acc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[h][a], b[h], acc[a], 0, 0, 0);
+        }
+    }
+    store_end_wgrad<4>(acc, kInRows, part + static_cast<size_t>(blockIdx.x) * (kInRows * 16));
+}
+// last layer: rows t of gy[v - off_t], columns ci of in[v][ci] (its BF16
+// input, exact in FP32); 996 us as thread-per-weight loops, 34 us so.
+__global__ void __launch_bounds__(256) k_conv_out_wgrad(Dims D, const uint16_t *__restrict__ in,
+                                                        const float *__restrict__ gy, float *__restrict__ part) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m0 = lane & 15, k = lane >> 4;
+    f32x4 acc[2];
+    int dx[2], dy[2], dz[2];
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+        tap_offset(a * 16 + m0 < 27 ? a * 16 + m0 : 13, dx[a], dy[a], dz[a]);
+    }
+    const int lines = D.Y * D.Z;
+    for (int line = blockIdx.x * 4 + wave; line < lines; line += 4 * static_cast<int>(gridDim.x)) {
+        const int y = line % D.Y, z = line / D.Y;
+        const float *src[2];
+        bool ok[2];
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            const int yy = y - dy[a], zz = z - dz[a];
+            ok[a] = a * 16 + m0 < 27 && yy >= 0 && yy < D.Y && zz >= 0 && zz < D.Z;
+            src[a] = gy + (ok[a] ? vox(D, 0, yy, zz) : 0);
+        }
+        const uint16_t *ir = in + vox(D, 0, y, z) * 16;
+        for (int i = 0; i < D.X; i += 8) {
+            float b[2], v[2][2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                b[h] = bf2f(ir[(i + 4 * h + k) * 16 + m0]);
+#pragma unroll
+                for (int a = 0; a < 2; a++) {
+                    const int xx = i + 4 * h + k - dx[a];
+                    const bool inside = ok[a] && xx >= 0 && xx < D.X;
+                    v[h][a] = src[a][inside ? xx : 0];
+                    v[h][a] = inside ? v[h][a] : 0.f;
+                }
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+                    acc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[h][a], b[h], acc[a], 0, 0, 0);
+        }
+    }
+    store_end_wgrad<2>(acc, 27, part + static_cast<size_t>(blockIdx.x) * (27 * 16));
 }
 
-// loss partials and dL/dy for the mean squared error over n voxels
-__global__ void k_mse(long long n, const float *__restrict__ y, const float *__restrict__ target,
-                      float *__restrict__ gy, float *__restrict__ loss) {
-    float s = 0.f;
+// Data gradient of the last layer, g[v][ci] = sum_t gy[v - off_t] W[t][ci]:
+// the skip gradient (FP32), its masked BF16 form and its channel sums.  The
+// FP32 matrix instruction with the weights as its rows, held in seven
+// registers over the whole launch (as scalar operands of vector
+// multiply-adds they were loaded again for every voxel: 31 us at 128x64x64
+// before the masked outputs and sums came in, 64 us with them); 21 us so.
+template <int CI>
+__global__ void __launch_bounds__(256) k_conv_out_dgrad(Dims D, const float *__restrict__ W,
+                                                        const float *__restrict__ gy, const uint16_t *__restrict__ act,
+                                                        float *__restrict__ gskip, uint16_t *__restrict__ gmask,
+                                                        float *__restrict__ part) {
+    static_assert(CI == 16, "one row tile");
+    constexpr int STEPS = 7;  // 27 taps in steps of four
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kg = lane >> 4;
+    float a[STEPS];
+    int dx[STEPS], dy[STEPS], dz[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+        const int t = 4 * s + kg;
+        a[s] = t < 27 ? W[t * CI + col] : 0.f;
+        tap_offset(t < 27 ? t : 13, dx[s], dy[s], dz[s]);
+    }
+    float4 sum{0.f, 0.f, 0.f, 0.f};
+    const int lines = D.Y * D.Z;
+    for (int line = blockIdx.x * 4 + wave; line < lines; line += 4 * static_cast<int>(gridDim.x)) {
+        const int y = line % D.Y, z = line / D.Y;
+        const float *src[STEPS];
+        bool ok[STEPS];
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) {
+            const int yy = y - dy[s], zz = z - dz[s];
+            ok[s] = yy >= 0 && yy < D.Y && zz >= 0 && zz < D.Z;
+            src[s] = gy + (ok[s] ? vox(D, 0, yy, zz) : 0);
+        }
+        for (int x0 = 0; x0 < D.X; x0 += 16) {
+            f32x4 acc{0.f, 0.f, 0.f, 0.f};
+            float b[STEPS];
+#pragma unroll
+            for (int s = 0; s < STEPS; s++) {
+                const int xx = x0 + col - dx[s];
+                const bool inside = ok[s] && xx >= 0 && xx < D.X;
+                b[s] = src[s][inside ? xx : 0];
+                b[s] = inside ? b[s] : 0.f;
+            }
+#pragma unroll
+            for (int s = 0; s < STEPS; s++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc, 0, 0, 0);
+            if (x0 + col >= D.X) continue;
+            const long long at = vox(D, x0 + col, y, z) * CI + 4 * kg;
+            *reinterpret_cast<float4 *>(gskip + at) = float4{acc[0], acc[1], acc[2], acc[3]};
+            const uint2 m = *reinterpret_cast<const uint2 *>(act + at);
+            float4 k;
+            k.x = positive(m.x & 0xFFFFu) ? acc[0] : 0.f;
+            k.y = positive(m.x >> 16) ? acc[1] : 0.f;
+            k.z = positive(m.y & 0xFFFFu) ? acc[2] : 0.f;
+            k.w = positive(m.y >> 16) ? acc[3] : 0.f;
+            *reinterpret_cast<uint2 *>(gmask + at) = uint2{pack2(k.x, k.y), pack2(k.z, k.w)};
+            sum.x += k.x;
+            sum.y += k.y;
+            sum.z += k.z;
+            sum.w += k.w;
+        }
+    }
+    __shared__ float s[4][CI];
+    float v[4] = {sum.x, sum.y, sum.z, sum.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        for (int off = 8; off > 0; off >>= 1) v[e] += __shfl_down(v[e], off, 16);
+        if (col == 0) s[wave][4 * kg + e] = v[e];
+    }
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < CI)
+        part[static_cast<size_t>(blockIdx.x) * CI + threadIdx.x] =
+            (s[0][threadIdx.x] + s[1][threadIdx.x]) + (s[2][threadIdx.x] + s[3][threadIdx.x]);
+}
+
+// dL/dy of the mean squared error over n voxels; per workgroup the sum of
+// (d^2) and of dL/dy (the last layer's bias gradient)
+__global__ void __launch_bounds__(256) k_mse(long long n, const float *__restrict__ y,
+                                             const float *__restrict__ target, float *__restrict__ gy,
+                                             float *__restrict__ part) {
+    float s = 0.f, b = 0.f;
     for (long long q = blockIdx.x * 256LL + threadIdx.x; q < n; q += 256LL * gridDim.x) {
-        const float d = y[q] - target[q];
-        gy[q] = 2.f * d / static_cast<float>(n);
+        const float d = y[q] - target[q], g = 2.f * d / static_cast<float>(n);
+        gy[q] = g;
         s += d * d;
+        b += g;
     }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(loss, s / static_cast<float>(n));
+    group_sums(float4{s, b, 0.f, 0.f}, 1, part + 4 * static_cast<size_t>(blockIdx.x));
 }
 
-// Adam on FP32 master weights; refreshes the BF16 copies in both layouts
-// ([t][ci][co] for the data gradient, [t][co][ci] for the forward pass).
-__global__ void k_adam(int n, int ci, int co, float *__restrict__ w, const float *__restrict__ g,
-                       float *__restrict__ m, float *__restrict__ v, float lr, float b1, float b2, float eps,
-                       float c1, float c2, uint16_t *__restrict__ w_bf, uint16_t *__restrict__ wt_bf) {
+// out[job][c] = scale * sum over the job's rows of part[row * stride + c], a
+// block of 64 columns per workgroup, its four wavefronts a quarter of the
+// rows each, added in a fixed order
+__global__ void __launch_bounds__(256) k_sum_rows(SumJobs J) {
+    int q = 0, first = 0;
+    for (; q < J.count - 1; q++) {
+        const int blocks = (J.job[q].n + 63) / 64;
+        if (static_cast<int>(blockIdx.x) < first + blocks) break;
+        first += blocks;
+    }
+    const SumJob &job = J.job[q];
+    const int c = (static_cast<int>(blockIdx.x) - first) * 64 + (threadIdx.x & 63), wave = threadIdx.x >> 6;
+    __shared__ float s[4][64];
+    float v = 0.f;
+    if (c < job.n) {
+        const int per = (job.rows + 3) / 4, r0 = wave * per, r1 = min(job.rows, r0 + per);
+#pragma unroll 8
+        for (int r = r0; r < r1; r++) v += job.part[static_cast<size_t>(r) * job.stride + c];
+    }
+    s[wave][threadIdx.x & 63] = v;
+    __syncthreads();
+    if (wave == 0 && c < job.n) {
+        const int l = threadIdx.x;
+        job.out[c] = job.scale * ((s[0][l] + s[1][l]) + (s[2][l] + s[3][l]));
+    }
+}
+
+// Adam on all FP32 master parameters
+__global__ void k_adam(int n, float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m,
+                       float *__restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    if (q >= n) return;
+    const float gq = g[q];
+    const float mq = b1 * m[q] + (1.f - b1) * gq;
+    const float vq = b2 * v[q] + (1.f - b2) * gq * gq;
+    m[q] = mq;
+    v[q] = vq;
+    w[q] = w[q] - lr * (mq / c1) / (sqrtf(vq / c2) + eps);
+}
+
+// The BF16 copies of every layer's weights in one launch (blockIdx.y: layer).
+// Plain layers: [27][ci][co] (data gradient) and [27][co][ci] (forward).
+// Upsampling layers, whose weights on the coarse input are sums: with the
+// fine taps t that meet on coarse tap t8 for output parity par (bits x, y, z
+// from the lowest) added in FP32 in tap order, `fwd` is [par][t8][co][ci]
+// (k_conv_fwd), rounded once, and `bwd` the sum of the BF16 weights as
+// [3 terms][64 fine offsets][ci][co] (k_conv_up_dgrad): coarse tap o at parity
+// p is the fine offset j = 3 - p - 2 o per axis, fine voxel 2 c - 1 + j.
+__global__ void k_weights_bf16(WeightJobs J) {
+    const WeightJob &l = J.job[blockIdx.y];
+    const int ci = l.ci, co = l.co, n = (l.up ? 64 : 27) * ci * co;
     for (int q = blockIdx.x * 256 + threadIdx.x; q < n; q += 256 * gridDim.x) {
-        const float gq = g[q];
-        const float mq = b1 * m[q] + (1.f - b1) * gq;
-        const float vq = b2 * v[q] + (1.f - b2) * gq * gq;
-        m[q] = mq;
-        v[q] = vq;
-        const float wq = w[q] - lr * (mq / c1) / (sqrtf(vq / c2) + eps);
-        w[q] = wq;
-        if (w_bf) {
+        if (!l.up) {
             const int t = q / (ci * co), r = q % (ci * co), i = r / co, o = r % co;
-            w_bf[q] = f2bf(wq);
-            wt_bf[(t * co + o) * ci + i] = f2bf(wq);
+            const uint16_t b = f2bf(l.w[q]);
+            l.bwd[q] = b;
+            l.fwd[(t * co + o) * ci + i] = b;
+            continue;
         }
-    }
-}
-
-// BF16 copies of FP32 weights in both layouts
-__global__ void k_weights_bf16(int n, int ci, int co, const float *__restrict__ w, uint16_t *__restrict__ w_bf,
-                               uint16_t *__restrict__ wt_bf) {
-    for (int q = blockIdx.x * 256 + threadIdx.x; q < n; q += 256 * gridDim.x) {
-        const int t = q / (ci * co), r = q % (ci * co), i = r / co, o = r % co;
-        w_bf[q] = f2bf(w[q]);
-        wt_bf[(t * co + o) * ci + i] = f2bf(w[q]);
-    }
-}
-
-// BF16 weights of the upsampling convolution's coarse form (k_conv_fwd):
-// wup[par][t8][o][i] = sum of W[t][i][o] over the fine taps t that meet on
-// coarse tap t8 for output parity par (bits x, y, z from the lowest), summed
-// in FP32 in tap order, rounded once
-__global__ void k_weights_up_bf16(int ci, int co, const float *__restrict__ w, uint16_t *__restrict__ wup) {
-    const int n = 64 * ci * co;
-    for (int q = blockIdx.x * 256 + threadIdx.x; q < n; q += 256 * gridDim.x) {
         const int i = q % ci, o = (q / ci) % co, t8 = (q / (ci * co)) % 8, par = q / (8 * ci * co);
         const int p[3] = {par & 1, (par >> 1) & 1, par >> 2}, oo[3] = {t8 & 1, (t8 >> 1) & 1, t8 >> 2};
-        float acc = 0.f;
+        float acc = 0.f, accb = 0.f;
         for (int t = 0; t < 27; t++) {
             int d[3];
             tap_offset(t, d[0], d[1], d[2]);
@@ -614,14 +934,21 @@ __global__ void k_weights_up_bf16(int ci, int co, const float *__restrict__ w, u
                 const int c = (p[a] + d[a] + 2) / 2 - 1;  // floor((p + d) / 2)
                 hit = hit && c == p[a] - 1 + oo[a];
             }
-            if (hit) acc += w[(t * ci + i) * co + o];
+            if (hit) {
+                const float w = l.w[(t * ci + i) * co + o];
+                acc += w;
+                accb += bf2f(f2bf(w));
+            }
         }
-        wup[q] = f2bf(acc);
+        l.fwd[q] = f2bf(acc);
+        const int jx = 3 - p[0] - 2 * oo[0], jy = 3 - p[1] - 2 * oo[1], jz = 3 - p[2] - 2 * oo[2];
+        const int at = ((jx + 4 * jy + 16 * jz) * ci + i) * co + o;
+        for (int h = 0; h < 3; h++) {
+            const uint16_t term = f2bf(accb);
+            l.bwd[64 * h * ci * co + at] = term;
+            accb -= bf2f(term);  // exact
+        }
     }
-}
-
-__global__ void k_fill_f(long long n, float *__restrict__ d, float v) {
-    for (long long q = blockIdx.x * 256LL + threadIdx.x; q < n; q += 256LL * gridDim.x) d[q] = v;
 }
 
 inline unsigned blocks_for(long long n) {
@@ -633,21 +960,23 @@ inline unsigned blocks_for(long long n) {
 
 // ---------------------------------------------------------------- launchers
 #define ARTSS_CONV_CASES(X) X(16, 16) X(16, 32) X(32, 64) X(64, 64) X(64, 32) X(32, 16)
+// voxels per wavefront row of k_conv_fwd: 16 x NV, eight matrix tiles per K step
+constexpr int row_tiles(int co) { return co == 16 ? 8 : (co == 32 ? 4 : 2); }
 
 void conv_fwd(hipStream_t s, int cin, int cout, bool up, Dims D, const uint16_t *in, const uint16_t *Wt,
               const float *bias, uint16_t *out, uint16_t *pre, const uint16_t *skip, bool relu) {
-    // voxels per wavefront row: 16 x NV with NV = 8, 4, 2 for 16, 32, 64
-    // output channels (8 matrix tiles per K step)
 #define CASE(CI, CO)                                                                                             \
     if (cin == CI && cout == CO) {                                                                              \
-        constexpr int NV = CO == 16 ? 8 : (CO == 32 ? 4 : 2);                                                    \
+        constexpr int NV = row_tiles(CO);                                                                       \
         const dim3 g((D.X + 16 * NV - 1) / (16 * NV), (D.Y + 3) / 4, D.Z);                                     \
         if (!up) {                                                                                              \
-            k_conv_fwd<CI, CO, false, NV><<<g, 256, 0, s>>>(D, in, Wt, bias, out, pre, skip, relu ? 1 : 0);     \
+            k_conv_fwd<CI, CO, false, NV>                                                                       \
+                <<<g, 256, 0, s>>>(D, in, Wt, bias, out, pre, skip, relu ? 1 : 0, nullptr);                     \
             return;                                                                                             \
         }                                                                                                       \
         if constexpr (CI >= 32) {                                                                               \
-            k_conv_fwd<CI, CO, true, NV><<<g, 256, 0, s>>>(D, in, Wt, bias, out, pre, skip, relu ? 1 : 0);      \
+            k_conv_fwd<CI, CO, true, NV>                                                                        \
+                <<<g, 256, 0, s>>>(D, in, Wt, bias, out, pre, skip, relu ? 1 : 0, nullptr);                     \
             return;                                                                                             \
         }                                                                                                       \
         throw std::invalid_argument("conv_fwd: an upsampled input needs at least 32 channels");               \
@@ -657,30 +986,66 @@ void conv_fwd(hipStream_t s, int cin, int cout, bool up, Dims D, const uint16_t 
     throw std::invalid_argument("conv_fwd: unsupported channel pair");
 }
 
-void conv_dgrad(hipStream_t s, int cin, int cout, Dims D, const float *gout, const uint16_t *W, float *gin) {
-    const dim3 g((D.X + 63) / 64, D.Y, D.Z);
-#define CASE(CI, CO)                                                      \
-    if (cin == CI && cout == CO) {                                       \
-        k_conv_dgrad<CI, CO><<<g, 256, 0, s>>>(D, gout, W, gin);         \
-        return;                                                          \
+void conv_dgrad(hipStream_t s, int cin, int cout, Dims D, const uint16_t *g, const uint16_t *W, const uint16_t *act,
+                float *gin) {
+#define CASE(CI, CO)                                                                                             \
+    if (cin == CI && cout == CO) {                                                                              \
+        constexpr int NV = row_tiles(CI);                                                                       \
+        const dim3 grid((D.X + 16 * NV - 1) / (16 * NV), (D.Y + 3) / 4, D.Z);                                  \
+        k_conv_fwd<CO, CI, false, NV, true>                                                                     \
+            <<<grid, 256, 0, s>>>(D, g, W, nullptr, nullptr, nullptr, act, 0, gin);                             \
+        return;                                                                                                 \
     }
-    ARTSS_CONV_CASES(CASE)
+    CASE(16, 16) CASE(16, 32) CASE(32, 64) CASE(64, 64)
 #undef CASE
     throw std::invalid_argument("conv_dgrad: unsupported channel pair");
 }
 
-void conv_wgrad(hipStream_t s, int cin, int cout, bool up, Dims D, const uint16_t *in, const float *gout,
-                float *gW) {
-    const int lines = D.Y * D.Z;
-    const int per = 16;
-    const dim3 g((lines + per - 1) / per, 27);
-#define CASE(CI, CO)                                                                            \
-    if (cin == CI && cout == CO) {                                                             \
-        if (up) k_conv_wgrad<CI, CO, true><<<g, 256, 0, s>>>(D, in, gout, gW, per);             \
-        else k_conv_wgrad<CI, CO, false><<<g, 256, 0, s>>>(D, in, gout, gW, per);               \
-        return;                                                                                \
+int up_dgrad_rows(int cin, int cout, Dims Dc) {
+    const int nv = cout == 64 ? 1 : (cin == 64 ? 2 : 4);
+    const long long tiles = static_cast<long long>((Dc.X + 16 * nv - 1) / (16 * nv)) * Dc.Y * Dc.Z;
+    return static_cast<int>(tiles < 1024 ? tiles : 1024);
+}
+void conv_up_dgrad(hipStream_t s, int cin, int cout, Dims Dc, const uint16_t *g, const uint16_t *Wd,
+                   const uint16_t *act, float *gskip, uint16_t *gmask, float *part) {
+    const unsigned rows = static_cast<unsigned>(up_dgrad_rows(cin, cout, Dc));
+    if (cin == 32 && cout == 16) k_conv_up_dgrad<16, 32, 4, 4, 2><<<rows, 256, 0, s>>>(Dc, g, Wd, act, gskip, gmask, part);
+    else if (cin == 64 && cout == 32)
+        k_conv_up_dgrad<32, 64, 2, 4, 4><<<rows, 256, 0, s>>>(Dc, g, Wd, act, gskip, gmask, part);
+    else if (cin == 64 && cout == 64)
+        k_conv_up_dgrad<64, 64, 1, 8, 1><<<dim3(rows, 4), 512, 0, s>>>(Dc, g, Wd, act, gskip, gmask, part);
+    else throw std::invalid_argument("conv_up_dgrad: unsupported channel pair");
+}
+
+// Partial rows of a weight gradient: enough workgroups (x 3 z offsets) to
+// fill the chip, few enough that the rows written and added again stay a
+// small part of the pass (27 ci co floats each).
+int wgrad_rows(int cin, int cout, Dims D) {
+    const int most = cin * cout <= 512 ? 256 : (cin * cout <= 2048 ? 96 : 32);
+    const int blocks = grad_blocks(D).blocks;
+    return blocks < most ? blocks : most;
+}
+void conv_wgrad(hipStream_t s, int cin, int cout, bool up, Dims D, const uint16_t *in, const uint16_t *g,
+                float *part) {
+    const GradBlocks B = grad_blocks(D);
+    const dim3 grid(static_cast<unsigned>(wgrad_rows(cin, cout, D)), 3);
+    const size_t fmax = static_cast<size_t>((B.rows * B.xb + 31) & ~31);
+    const size_t pos = up ? static_cast<size_t>(B.rows / 2 + 2) * ((B.xb + 1) / 2 + 2)
+                          : static_cast<size_t>(B.rows + 2) * (B.xb + 2);
+#define CASE(CI, CO, UP)                                                                                       \
+    if (cin == CI && cout == CO && up == UP) {                                                                \
+        const size_t bytes = 2 * (fmax * lds_voxel<CO>() + pos * lds_voxel<CI>());                            \
+        /* at most (2 + 2) x (128 + 2) halo voxels and 256 others: 121 KB at 64 channels */                   \
+        if (bytes > 64 * 1024 &&                                                                              \
+            hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv_wgrad<CI, CO, UP>),                    \
+                                hipFuncAttributeMaxDynamicSharedMemorySize,                                   \
+                                static_cast<int>(bytes)) != hipSuccess)                                       \
+            throw std::runtime_error("conv_wgrad: the block does not fit in this device's LDS");              \
+        k_conv_wgrad<CI, CO, UP><<<grid, 192, bytes, s>>>(D, B, in, g, part);                                 \
+        return;                                                                                               \
     }
-    ARTSS_CONV_CASES(CASE)
+    CASE(16, 16, false) CASE(16, 32, false) CASE(32, 64, false) CASE(64, 64, false)
+    CASE(64, 64, true) CASE(64, 32, true) CASE(32, 16, true)
 #undef CASE
     throw std::invalid_argument("conv_wgrad: unsupported channel pair");
 }
@@ -691,19 +1056,36 @@ void conv_in(hipStream_t s, Dims D, const float *x, const float *W, const float 
 void conv_out(hipStream_t s, Dims D, const uint16_t *in, const float *W, const float *bias, float *y) {
     k_conv_out<16, 8><<<dim3((D.X + 63) / 64, (D.Y + 3) / 4, (D.Z + 7) / 8), dim3(64, 4, 1), 0, s>>>(D, in, W, bias, y);
 }
-void conv_in_wgrad(hipStream_t s, Dims D, const float *x, const float *g, float *gW, float *gb) {
-    const long long n = static_cast<long long>(D.X) * D.Y * D.Z;
-    const long long per = 2048;
-    k_conv_in_wgrad<2, 16><<<static_cast<unsigned>((n + per - 1) / per), 27 * 2 * 16, 0, s>>>(D, x, g, gW, per);
-    bias_grad(s, 16, n, g, gb);
+// one workgroup per four x rows, at most two per CU
+int end_wgrad_rows(Dims D) {
+    const long long lines = static_cast<long long>(D.Y) * D.Z;
+    return static_cast<int>(lines < 4 * 512 ? (lines + 3) / 4 : 512);
 }
-void conv_out_grads(hipStream_t s, Dims D, const uint16_t *in, const float *W, const float *gy, float *gW,
-                    float *gb, float *gin) {
-    const long long n = static_cast<long long>(D.X) * D.Y * D.Z;
-    const long long per = 2048;
-    k_conv_out_wgrad<16><<<static_cast<unsigned>((n + per - 1) / per), 27 * 16, 0, s>>>(D, in, gy, gW, per);
-    k_conv_out_dgrad<16><<<blocks_for(n), 256, 0, s>>>(D, W, gy, gin);
-    bias_grad(s, 1, n, gy, gb);
+void conv_in_wgrad(hipStream_t s, Dims D, const float *x, const float *g, float *part) {
+    k_conv_in_wgrad<<<static_cast<unsigned>(end_wgrad_rows(D)), 256, 0, s>>>(D, x, g, part);
+}
+void conv_out_wgrad(hipStream_t s, Dims D, const uint16_t *in, const float *gy, float *part) {
+    k_conv_out_wgrad<<<static_cast<unsigned>(end_wgrad_rows(D)), 256, 0, s>>>(D, in, gy, part);
+}
+int end_dgrad_rows(Dims D) {
+    const long long lines = static_cast<long long>(D.Y) * D.Z;
+    return static_cast<int>(lines < 4 * 1024 ? (lines + 3) / 4 : 1024);
+}
+int elementwise_rows(long long voxels, int groups) {
+    const long long b = (voxels * groups + 1023) / 1024;  // four items per thread
+    return static_cast<int>(b < 1 ? 1 : (b > 512 ? 512 : b));
+}
+void conv_out_dgrad(hipStream_t s, Dims D, const float *W, const float *gy, const uint16_t *act, float *gskip,
+                    uint16_t *gmask, float *part) {
+    k_conv_out_dgrad<16><<<static_cast<unsigned>(end_dgrad_rows(D)), 256, 0, s>>>(D, W, gy, act, gskip, gmask, part);
+}
+void enc_grad(hipStream_t s, int c, Dims D, const float *gskip, const float *gc, const uint16_t *act, uint16_t *gmask,
+              float *part) {
+    const unsigned b = static_cast<unsigned>(elementwise_rows(static_cast<long long>(D.X) * D.Y * D.Z, c / 4));
+    if (c == 16) k_enc_grad<16><<<b, 256, 0, s>>>(D, gskip, gc, act, gmask, part);
+    else if (c == 32) k_enc_grad<32><<<b, 256, 0, s>>>(D, gskip, gc, act, gmask, part);
+    else if (c == 64) k_enc_grad<64><<<b, 256, 0, s>>>(D, gskip, gc, act, gmask, part);
+    else throw std::invalid_argument("enc_grad: unsupported channels");
 }
 void down(hipStream_t s, int c, Dims Dc, const uint16_t *in, uint16_t *out) {
     const long long n = static_cast<long long>(Dc.X) * Dc.Y * Dc.Z * c;
@@ -712,48 +1094,20 @@ void down(hipStream_t s, int c, Dims Dc, const uint16_t *in, uint16_t *out) {
     else if (c == 64) k_down<64><<<blocks_for(n), 256, 0, s>>>(Dc, in, out);
     else throw std::invalid_argument("down: unsupported channels");
 }
-void down_backward_add(hipStream_t s, int c, Dims Dc, const float *gc, float *gf) {
-    const long long n = static_cast<long long>(Dc.X) * Dc.Y * Dc.Z * 8 * c;
-    if (c == 16) k_down_backward_add<16><<<blocks_for(n), 256, 0, s>>>(Dc, gc, gf);
-    else if (c == 32) k_down_backward_add<32><<<blocks_for(n), 256, 0, s>>>(Dc, gc, gf);
-    else if (c == 64) k_down_backward_add<64><<<blocks_for(n), 256, 0, s>>>(Dc, gc, gf);
-    else throw std::invalid_argument("down_backward_add: unsupported channels");
+void mse(hipStream_t s, long long n, const float *y, const float *target, float *gy, float *part) {
+    k_mse<<<static_cast<unsigned>(elementwise_rows(n, 1)), 256, 0, s>>>(n, y, target, gy, part);
 }
-void up_backward(hipStream_t s, int c, Dims Dc, const float *gf, float *gc) {
-    const long long n = static_cast<long long>(Dc.X) * Dc.Y * Dc.Z * c;
-    if (c == 16) k_up_backward<16><<<blocks_for(n), 256, 0, s>>>(Dc, gf, gc);
-    else if (c == 32) k_up_backward<32><<<blocks_for(n), 256, 0, s>>>(Dc, gf, gc);
-    else if (c == 64) k_up_backward<64><<<blocks_for(n), 256, 0, s>>>(Dc, gf, gc);
-    else throw std::invalid_argument("up_backward: unsupported channels");
+void sum_rows(hipStream_t s, const SumJobs &jobs) {
+    unsigned blocks = 0;
+    for (int q = 0; q < jobs.count; q++) blocks += static_cast<unsigned>((jobs.job[q].n + 63) / 64);
+    if (blocks) k_sum_rows<<<blocks, 256, 0, s>>>(jobs);
 }
-void bias_grad(hipStream_t s, int c, long long voxels, const float *g, float *gb) {
-    const unsigned b = blocks_for(voxels) > 512 ? 512 : blocks_for(voxels);
-    if (c == 1) k_bias_grad<1><<<b, 256, 0, s>>>(voxels, g, gb);
-    else if (c == 16) k_bias_grad<16><<<b, 256, 0, s>>>(voxels, g, gb);
-    else if (c == 32) k_bias_grad<32><<<b, 256, 0, s>>>(voxels, g, gb);
-    else if (c == 64) k_bias_grad<64><<<b, 256, 0, s>>>(voxels, g, gb);
-    else throw std::invalid_argument("bias_grad: unsupported channels");
+void adam(hipStream_t s, int n, float *w, const float *g, float *m, float *v, float lr, float b1, float b2, float eps,
+          float c1, float c2) {
+    k_adam<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(n, w, g, m, v, lr, b1, b2, eps, c1, c2);
 }
-void relu_mask(hipStream_t s, long long n, float *g, const uint16_t *act) {
-    k_relu_mask<<<blocks_for(n), 256, 0, s>>>(n, g, act);
-}
-void copy_f(hipStream_t s, long long n, float *dst, const float *src) {
-    k_copy_f<<<blocks_for(n), 256, 0, s>>>(n, dst, src);
-}
-void fill_f(hipStream_t s, long long n, float *dst, float v) { k_fill_f<<<blocks_for(n), 256, 0, s>>>(n, dst, v); }
-void mse(hipStream_t s, long long n, const float *y, const float *target, float *gy, float *loss) {
-    k_mse<<<blocks_for(n) > 1024 ? 1024 : blocks_for(n), 256, 0, s>>>(n, y, target, gy, loss);
-}
-void adam(hipStream_t s, int n, int ci, int co, float *w, const float *g, float *m, float *v, float lr, float b1,
-          float b2, float eps, float c1, float c2, uint16_t *w_bf, uint16_t *wt_bf) {
-    k_adam<<<blocks_for(n), 256, 0, s>>>(n, ci, co, w, g, m, v, lr, b1, b2, eps, c1, c2, w_bf, wt_bf);
-}
-void weights_up_bf16(hipStream_t s, int ci, int co, const float *w, uint16_t *wup) {
-    k_weights_up_bf16<<<blocks_for(64LL * ci * co), 256, 0, s>>>(ci, co, w, wup);
-}
-
-void weights_bf16(hipStream_t s, int n, int ci, int co, const float *w, uint16_t *w_bf, uint16_t *wt_bf) {
-    k_weights_bf16<<<blocks_for(n), 256, 0, s>>>(n, ci, co, w, w_bf, wt_bf);
+void weights_bf16(hipStream_t s, const WeightJobs &jobs) {
+    if (jobs.count) k_weights_bf16<<<dim3(256, static_cast<unsigned>(jobs.count)), 256, 0, s>>>(jobs);
 }
 
 }  // namespace nn
