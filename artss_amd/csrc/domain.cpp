@@ -134,7 +134,8 @@ Domain::Domain(const Settings &s, int device) : m_settings(s), m_device(device) 
     m_partial_cap = 1;
     for (int l = 0; l <= m_levels; l++) m_partial_cap = std::max(m_partial_cap, k::partial_count(m_level[l]));
     ARTSS_HIP(hipMalloc(&m_partial, sizeof(double) * static_cast<size_t>(m_partial_cap)));
-    ARTSS_HIP(hipMalloc(&m_sum_dev, sizeof(double)));
+    ARTSS_HIP(hipMalloc(&m_gate, sizeof(k::IterGate)));
+    ARTSS_HIP(hipHostMalloc(&m_gate_host, sizeof(k::IterGate), hipHostMallocDefault));
     ARTSS_HIP(hipHostMalloc(&m_sum_host, sizeof(double), hipHostMallocDefault));
     static_scratch_setup(device);
 }
@@ -144,7 +145,8 @@ Domain::~Domain() {
     timer_clear();
     (void)hipStreamSynchronize(m_stream);
     (void)hipFree(m_partial);
-    (void)hipFree(m_sum_dev);
+    (void)hipFree(m_gate);
+    (void)hipHostFree(m_gate_host);
     (void)hipHostFree(m_sum_host);
     (void)hipFree(m_faces_dev);
     (void)hipFree(m_params_dev);
@@ -683,8 +685,7 @@ void Domain::apply_faces(double *f, int ft, int level) {
 
 void Domain::reduce_async(const double *partial, int n) {
     require_device();
-    k::reduce_sum(m_stream, partial, n, m_sum_dev);
-    ARTSS_HIP(hipMemcpyAsync(m_sum_host, m_sum_dev, sizeof(double), hipMemcpyDeviceToHost, m_stream));
+    k::reduce_sum(m_stream, partial, n, m_sum_host);
 }
 
 double Domain::reduce(const double *partial, int n) {

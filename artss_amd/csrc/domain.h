@@ -30,6 +30,10 @@ class hip_error : public std::runtime_error {
 void hip_check(hipError_t e, const char *what);
 #define ARTSS_HIP(call) ::artss::hip_check((call), #call)
 
+namespace k {
+struct IterGate;
+}
+
 struct ObstacleLevel {
     size_t start[3], end[3];
     std::vector<uint64_t> face[6];  // Obstacle::m_boundary per patch, sorted
@@ -118,6 +122,10 @@ class Domain {
     // with reduced_value() once the stream has been synchronised
     void reduce_async(const double *partial, int n);
     double reduced_value() const { return *m_sum_host; }
+    // device loop state of the diffusion iterations and its pinned mirror
+    // (one loop at a time: a domain's calls run in order on its stream)
+    k::IterGate *loop_gate() const { return m_gate; }
+    k::IterGate *loop_mirror() const { return m_gate_host; }
     double *partial_buffer() const { return m_partial; }
     int partial_capacity() const { return m_partial_cap; }
 
@@ -204,8 +212,8 @@ class Domain {
 
     double *m_partial = nullptr;
     int m_partial_cap = 0;
-    double *m_sum_dev = nullptr;
-    double *m_sum_host = nullptr;
+    double *m_sum_host = nullptr;  // pinned; the reduction writes it from the device
+    k::IterGate *m_gate = nullptr, *m_gate_host = nullptr;
 
     void require_device() const;
     void build_levels();

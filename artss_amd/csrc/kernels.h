@@ -90,6 +90,13 @@ void cgs_iter(hipStream_t s, const LevelDesc &L, const BCView &V, const CgsCoef 
               const double *src, double *dst, double *partial, const int *gate);
 // exchanges the contents of two arrays of n values
 void swap_arrays(hipStream_t s, double *a, double *b, long long n);
+// One Jacobi diffusion iteration in one launch (the sweep from src to dst,
+// the fill, norm partials; a fill that is idempotent): src and dst are `in`
+// and `out` in turn, starting from `in`.
+int jacobi_iter_partials(const LevelDesc &L, const BCView &V);
+void jacobi_iter(hipStream_t s, const LevelDesc &L, const BCView &V, double *dst, const double *src, const double *in,
+                 const double *out, const double *b, double ax, double ay, double az, double rb, double D,
+                 const double *ev, double dt, double w, double *partial, const int *gate);
 
 // ---- multigrid (VCycleMG.cpp) ----
 void residuum(hipStream_t s, const LevelDesc &L, double *out, const double *x, const double *b);   // :346-354
@@ -156,7 +163,8 @@ void log_gate(hipStream_t s, const IterGate *g, LoopLog *log);
 void alternate_finish(hipStream_t s, const IterGate *g, double *out, double *in, long long n);
 // reduce_sum into g->sum, then count the iteration and set done as the
 // loop `while (sqrt(sum) > tol && count < max_iter)` decides; nothing once done
-void reduce_gate(hipStream_t s, const double *partial, int n, IterGate *g);
+// (mirror, optional: pinned host memory that receives sum, count and done)
+void reduce_gate(hipStream_t s, const double *partial, int n, IterGate *g, IterGate *mirror = nullptr);
 
 // ---- DynamicSmagorinsky (turbulence/DynamicSmagorinsky.cpp) ----
 constexpr int kDynMax = 12;

@@ -593,33 +593,39 @@ __device__ __forceinline__ double cgs_update(const LevelDesc &L, const CgsCoef &
 // fill writes: the previous fill).
 //
 // A workgroup of kCgsWaves wavefronts owns a tile of kCgsOwnX x kCgsOwnY
-// columns (i, j) and marches along z through kCgsPlanes planes.  Each lane
+// columns (i, j) and marches along z through T.planes planes.  Each lane
 // holds two cells adjacent along x, so that every lane updates one cell of
 // each colour per plane; a wavefront covers two rows of 64 cells, and the
 // tile has a one-cell halo of columns and rows.  At step t each lane
-// evaluates the first colour at plane t + 1 (src from memory) and puts the
-// values its two cells hold after the first colour into a three-plane ring
-// in LDS; after one barrier it updates the second colour at plane t from
-// the ring (x, y) and its own registers (z), writes dst, applies the fill
-// through its face ghosts and adds the update norm.  Fill items run in
-// extra workgroups that re-evaluate both colours from src at the cell each
-// write reads.
+// evaluates the first colour at plane t + 1 and puts the value that cell
+// holds after the first colour into a three-plane ring in LDS; after one
+// barrier it updates the second colour at plane t, whose six neighbours are
+// all first-colour cells (from the ring along y and outward along x, from its
+// own registers along z and inward), writes dst, applies the fill through its
+// face ghosts and adds the update norm.  Fill items run in extra workgroups
+// that re-evaluate both colours from src at the cell each write reads.
+//
+// What bounds it is the latency of a step (loads, a barrier, two divisions)
+// times the planes a workgroup marches through, at four wavefronts per SIMD.
+// So a lane carries src, b, the eddy viscosity and the first colour's
+// coefficient from plane to plane (three 16-byte and three 8-byte loads per
+// step; reloading them took fifteen), and the loads of step t + 1 are issued
+// before step t computes.
 //
 // Memory is read through buffer descriptors with 32-bit offsets: a load
 // outside an array returns 0 instead of touching memory, so every lane
 // issues the same loads at every step, whatever cells it holds, with no
 // branch around them (a value read outside its array reaches no update:
 // the neighbours of a fluid cell lie inside the array).
-// (4 wavefronts and 16 planes measured fastest on the 256x128x128 plume:
-// 71.5 us per iteration against 73.9 for 8 wavefronts, 81.9 for 8 planes)
 constexpr int kCgsWaves = 4;
 constexpr int kCgsRows = 2 * kCgsWaves;  // rows of a tile with its halo
 constexpr int kCgsOwnX = 62;             // of 64 cells per row
 constexpr int kCgsOwnY = kCgsRows - 2;
-constexpr int kCgsPlanes = 16;
+constexpr int kCgsItemLanes = 8;         // lanes per fill item
 
 struct CgsTiles {
     int tx, ty, tz;  // tiles along x, y and z; main workgroups tx * ty * tz
+    int planes;      // planes of a tile
 };
 
 __device__ __forceinline__ bool fluid_at(const LevelDesc &L, int i, int j, int k) {
@@ -643,6 +649,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, unsig
 __device__ __forceinline__ double buffer_f64(__amdgpu_buffer_rsrc_t r, unsigned offset) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, offset, 0, 0));
 }
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ f64x2 buffer_f64x2(__amdgpu_buffer_rsrc_t r, unsigned offset) {
+    return __builtin_bit_cast(f64x2, __builtin_amdgcn_raw_buffer_load_b128(r, offset, 0, 0));
+}
 __device__ __forceinline__ unsigned buffer_u32(__amdgpu_buffer_rsrc_t r, unsigned offset) {
     return __builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, 0);
 }
@@ -656,27 +666,25 @@ __global__ void __launch_bounds__(64 * kCgsWaves)
     const unsigned main_blocks = static_cast<unsigned>(T.tx) * T.ty * T.tz;
     const long long nj = L.N[0], nk = static_cast<long long>(L.N[0]) * L.N[1];
     if (blockIdx.x >= main_blocks) {
-        // fill items: the value the iteration gives the cell each write reads
-        const long long t = static_cast<long long>(blockIdx.x - main_blocks) * (64 * kCgsWaves) + threadIdx.y * 64 +
-                            threadIdx.x;
+        // Fill items: the value the iteration gives the cell each write reads.
+        // Eight lanes share an item, so that the six first-colour neighbours
+        // of a second-colour cell are evaluated side by side (one after the
+        // other, their latency set the launch's length on small levels: 18 us
+        // at 64x64x32 whatever the tiles, 12 us so).
+        const long long t =
+            (static_cast<long long>(blockIdx.x - main_blocks) * (64 * kCgsWaves) + threadIdx.y * 64 + threadIdx.x) /
+            kCgsItemLanes;
+        const int sub = static_cast<int>(threadIdx.x) % kCgsItemLanes;
         auto val = [&](long long q) -> double {
             int i, j, k;
             if (!is_inner(L, q, i, j, k)) return src[q];
             if (((i + j + k) & 1) == 0) return cgs_update(L, c, ev, src, src, b, q, nullptr);
-            // the six neighbours after the first colour (one evaluation in a
-            // loop keeps the item code small)
+            const int d = sub < 6 ? sub : 0;
+            const long long step = (d >> 1) == 0 ? 1 : ((d >> 1) == 1 ? nj : nk);
+            const double x = cgs_first(L, c, ev, b, src, (d & 1) ? q - step : q + step);
             double nb[6];
-#pragma unroll 1
-            for (int d = 0; d < 6; d++) {
-                const long long step = (d >> 1) == 0 ? 1 : ((d >> 1) == 1 ? nj : nk);
-                const double x = cgs_first(L, c, ev, b, src, (d & 1) ? q - step : q + step);
-                nb[0] = d == 0 ? x : nb[0];
-                nb[1] = d == 1 ? x : nb[1];
-                nb[2] = d == 2 ? x : nb[2];
-                nb[3] = d == 3 ? x : nb[3];
-                nb[4] = d == 4 ? x : nb[4];
-                nb[5] = d == 5 ? x : nb[5];
-            }
+#pragma unroll
+            for (int e = 0; e < 6; e++) nb[e] = __shfl(x, e, kCgsItemLanes);
             return cgs_value(c, ev, q, src[q], nb[0], nb[1], nb[2], nb[3], nb[4], nb[5], b[q], nullptr);
         };
         dev::bc_item<double, decltype(val), true>(L, V, t, dst, val);
@@ -697,8 +705,8 @@ __global__ void __launch_bounds__(64 * kCgsWaves)
     const bool own_row = r >= 1 && r <= kCgsOwnY && j >= 0 && j < L.N[1];
     const bool own_a = own_row && pr >= 1 && xa >= 0 && xa < L.N[0];
     const bool own_b = own_row && pr <= 30 && xa + 1 >= 0 && xa + 1 < L.N[0];
-    const int k0 = tz * kCgsPlanes;
-    const int k1 = min(k0 + kCgsPlanes, L.N[2]);
+    const int k0 = tz * T.planes;
+    const int k1 = min(k0 + T.planes, L.N[2]);
     constexpr bool turb = TURB;
     // columns of the two cells: inside the inner box, and inside each obstacle's x-y extent (bit o)
     const bool in_a = xa >= 1 && xa <= L.n[0] && j >= 1 && j <= L.n[1];
@@ -723,113 +731,102 @@ __global__ void __launch_bounds__(64 * kCgsWaves)
     // byte offset of cell xa of row j in plane 0 (wraps for cells before the array)
     const unsigned lo = static_cast<unsigned>(xa + static_cast<int>(nj) * j) * 8u;
     const unsigned pn = static_cast<unsigned>(nk) * 8u, rn = static_cast<unsigned>(nj) * 8u;
-    __shared__ double ring[3][kCgsRows][64];
-    // every value step t reads from memory (cells xa, xa + 1; slot s of the
-    // pair is the first-colour cell at plane t + 1 and the second-colour
-    // cell at plane t, the same one): src of both cells at planes t and t + 1;
-    // at the slot's cell src at plane t + 2, its outer x neighbour and its
-    // y neighbours at t + 1, b and the eddy viscosity at t + 1, b at t; the
-    // eddy viscosity of both cells and the fill's bits at t
+    __shared__ double ring[3][kCgsRows][32];
+    // "slot": the lane's cell (a when sa) that is first colour at plane t + 1
+    // and second colour at plane t.  Per step, from memory: src of both cells
+    // at plane t + 2; b and the eddy viscosity of both at t + 1; the slot's
+    // outer x neighbour and y neighbours at t + 1; the fill's bits at t (both
+    // cells in one word: xa and the row length are even)
     struct Fetch {
-        double s0a, s0b, s1a, s1b, s2, xo, yp, ym, bn, en, bc, eca, ecb;
-        unsigned wa, wb;
+        f64x2 s2, b1, e1;
+        double xo, yp, ym;
+        unsigned w;
     };
     auto fetch = [&](int t) -> Fetch {
         const unsigned o0 = lo + static_cast<unsigned>(t) * pn, o1 = o0 + pn, o2 = o1 + pn;
-        const bool sa = ((j + t) & 1) == 1;  // slot 0 (cell xa)
+        const bool sa = ((j + t) & 1) == 1;
         const unsigned e = sa ? 0u : 8u;
-        const unsigned ca = o0 / 8u;  // cell index of xa at plane t (wrapped when outside)
         Fetch f;
-        f.s0a = buffer_f64(rs, o0);
-        f.s0b = buffer_f64(rs, o0 + 8u);
-        f.s1a = buffer_f64(rs, o1);
-        f.s1b = buffer_f64(rs, o1 + 8u);
-        f.s2 = buffer_f64(rs, o2 + e);
+        f.s2 = buffer_f64x2(rs, o2);
+        f.b1 = buffer_f64x2(rb_, o1);
+        f.e1 = TURB ? buffer_f64x2(re, o1) : f64x2{0.0, 0.0};
         f.xo = buffer_f64(rs, sa ? o1 - 8u : o1 + 16u);
         f.yp = buffer_f64(rs, o1 + e + rn);
         f.ym = buffer_f64(rs, o1 + e - rn);
-        f.bn = buffer_f64(rb_, o1 + e);
-        f.en = TURB ? buffer_f64(re, o1 + e) : 0.0;
-        f.bc = buffer_f64(rb_, o0 + e);
-        f.eca = TURB ? buffer_f64(re, o0) : 0.0;
-        f.ecb = TURB ? buffer_f64(re, o0 + 8u) : 0.0;
-        f.wa = buffer_u32(rw, (ca >> 5) * 4u);
-        f.wb = buffer_u32(rw, ((ca + 1u) >> 5) * 4u);
+        f.w = buffer_u32(rw, (o0 >> 8) * 4u);
         return f;
     };
-    // the two cells' values after the first colour at planes t - 1 and t
-    double pa = 0.0, pb = 0.0, ma = 0.0, mb = 0.0;
-    double sq = 0.0;
-    auto rb_of = [&](double e) {
-        return turb ? (1. + 2. * ((c.D + e) * c.dt * c.rdx * c.rdx + (c.D + e) * c.dt * c.rdy * c.rdy +
-                                  (c.D + e) * c.dt * c.rdz * c.rdz))
-                    : c.rb;
-    };
-    // step t with the loads fetched for it
-    auto step = [&](int t, const Fetch &f) {
+    // planes t and t + 1 of src; b and the viscosity at t; the two cells'
+    // values after the first colour at t - 1 (pa, pb) and t (ma, mb); the
+    // coefficient 1 + 2 (aX + aY + aZ) of the first-colour cell at t
+    const int t0 = k0 - 2;
+    f64x2 s0 = buffer_f64x2(rs, lo + static_cast<unsigned>(t0) * pn),
+          s1 = buffer_f64x2(rs, lo + static_cast<unsigned>(t0 + 1) * pn), b0{0.0, 0.0}, e0{0.0, 0.0};
+    double pa = 0.0, pb = 0.0, ma = 0.0, mb = 0.0, rb0 = c.rb, sq = 0.0;
+    Fetch f = fetch(t0);
+    for (int t = t0; t < k1; t++) {
+        const Fetch next = fetch(t + 1);
         // first colour at plane t + 1: the slot's cell
         const int kn = t + 1;
         const bool kin = kn >= 1 && kn <= L.n[2];
-        const unsigned zm = zmask(kn);
-        const bool sa = ((j + t) & 1) == 1;  // slot 0: xa + j + t + 1 even
-        const bool fl = sa ? (in_a && kin && (ob_a & zm) == 0) : (in_b && kin && (ob_b & zm) == 0);
-        double na = f.s1a, nb = f.s1b;
-        if (fl) {
-            const double v = cgs_value_e(c, turb, f.en, sa ? f.s1a : f.s1b, sa ? f.s1b : f.xo, sa ? f.xo : f.s1a,
-                                         f.yp, f.ym, f.s2, sa ? f.s0a : f.s0b, f.bn, nullptr);
-            na = sa ? v : na;
-            nb = sa ? nb : v;
+        const bool sa = ((j + t) & 1) == 1;  // cell a: xa + j + t + 1 even
+        const bool fl = (sa ? in_a : in_b) && kin && ((sa ? ob_a : ob_b) & zmask(kn)) == 0;
+        double nv = sa ? s1.x : s1.y, rb1;
+        {
+            const double other = sa ? s1.y : s1.x;
+            const double v = cgs_value_e(c, turb, sa ? f.e1.x : f.e1.y, nv, sa ? other : f.xo, sa ? f.xo : other, f.yp,
+                                         f.ym, sa ? f.s2.x : f.s2.y, sa ? s0.x : s0.y, sa ? f.b1.x : f.b1.y, &rb1);
+            nv = fl ? v : nv;
         }
-        double *slot = &ring[(t + 4) % 3][r][2 * pr];
-        slot[0] = na;
-        slot[1] = nb;
+        const double na = sa ? nv : s1.x, nb = sa ? s1.y : nv;
+        ring[(t + 4) % 3][r][pr] = nv;
         __syncthreads();
         // second colour, fill and norm at plane t: the slot's cell
-        if (t >= k0 && t < k1 && (own_a || own_b)) {
+        if (t >= k0 && (own_a || own_b)) {
             const bool tin = t >= 1 && t <= L.n[2];
             const unsigned zc = zmask(t);
             const bool fa = own_a && in_a && tin && (ob_a & zc) == 0;
             const bool fb = own_b && in_b && tin && (ob_b & zc) == 0;
             const int q = (t + 3) % 3;
-            double fin_a = ma, fin_b = mb, rba, rbb;
+            double fin_a = ma, fin_b = mb, rbs = rb0;
             if (sa ? fa : fb) {
-                const int x = 2 * pr + (sa ? 0 : 1);  // column of the tile
-                double rbs;
-                const double v = cgs_value_e(c, turb, sa ? f.eca : f.ecb, sa ? f.s0a : f.s0b, ring[q][r][x + 1],
-                                             ring[q][r][x - 1], ring[q][r + 1][x], ring[q][r - 1][x],
-                                             sa ? na : nb, sa ? pa : pb, f.bc, &rbs);
+                // inward along x the lane's other cell, outward the next lane's
+                const double in_x = sa ? mb : ma, out_x = ring[q][r][sa ? pr - 1 : pr + 1];
+                const double v = cgs_value_e(c, turb, sa ? e0.x : e0.y, sa ? s0.x : s0.y, sa ? in_x : out_x,
+                                             sa ? out_x : in_x, ring[q][r + 1][pr], ring[q][r - 1][pr], nv,
+                                             sa ? pa : pb, sa ? b0.x : b0.y, &rbs);
                 fin_a = sa ? v : fin_a;
                 fin_b = sa ? fin_b : v;
-                rba = sa ? rbs : rb_of(f.eca);
-                rbb = sa ? rb_of(f.ecb) : rbs;
-            } else {
-                rba = rb_of(f.eca);
-                rbb = rb_of(f.ecb);
             }
             const long long ia = static_cast<long long>(xa) + nj * j + nk * t;
             if (fa) {
                 dst[ia] = fin_a;
                 dev::face_ghosts(L, V, dst, ia, xa, j, t, fin_a);
-                const double d = rba * (fin_a - f.s0a);
+                const double d = (sa ? rbs : rb0) * (fin_a - s0.x);
                 sq += d * d;
-            } else if (own_a && ((f.wa >> (static_cast<unsigned>(ia) & 31u)) & 1u) == 0) {
-                dst[ia] = f.s0a;  // not written by the fill
+            } else if (own_a && ((f.w >> (static_cast<unsigned>(ia) & 31u)) & 1u) == 0) {
+                dst[ia] = s0.x;  // not written by the fill
             }
             if (fb) {
                 dst[ia + 1] = fin_b;
                 dev::face_ghosts(L, V, dst, ia + 1, xa + 1, j, t, fin_b);
-                const double d = rbb * (fin_b - f.s0b);
+                const double d = (sa ? rb0 : rbs) * (fin_b - s0.y);
                 sq += d * d;
-            } else if (own_b && ((f.wb >> (static_cast<unsigned>(ia + 1) & 31u)) & 1u) == 0) {
-                dst[ia + 1] = f.s0b;
+            } else if (own_b && ((f.w >> (static_cast<unsigned>(ia + 1) & 31u)) & 1u) == 0) {
+                dst[ia + 1] = s0.y;
             }
         }
         pa = ma;
         pb = mb;
         ma = na;
         mb = nb;
-    };
-    for (int t = k0 - 2; t < k1; t++) step(t, fetch(t));
+        s0 = s1;
+        s1 = f.s2;
+        b0 = f.b1;
+        e0 = f.e1;
+        rb0 = rb1;
+        f = next;
+    }
     // workgroup sum in a fixed order
     for (int off = 32; off > 0; off >>= 1) sq += __shfl_down(sq, off, 64);
     __shared__ double wsum[kCgsWaves];
@@ -842,10 +839,125 @@ __global__ void __launch_bounds__(64 * kCgsWaves)
     }
 }
 
+// Planes per tile: the most (16, 8, 4 or 2) that still give kCgsFill
+// workgroups.  Every tile evaluates two planes besides its own, so deep tiles
+// do less work, but a launch that leaves the chip short of wavefronts takes
+// as long as one workgroup's march.  Measured, us per iteration with 16 / 8 /
+// 4 / 2 planes: 256x128x128 (990 workgroups at 16) 52 / 57 / 62 / 66;
+// 128x128x128 (594) 42 / 41 / 41 / 45; 160x96x64 (255) 29 / 22 / 22 / 23;
+// 112x80x48 (112) 29 / 19 / 16 / 14; 32x32x32 (18) 30 / 20 / 13 / 11.
+constexpr int kCgsFill = 512;
 inline CgsTiles cgs_tiles(const LevelDesc &L) {
     // tile tx owns columns tx * kCgsOwnX - 1 .. tx * kCgsOwnX + 60
-    return CgsTiles{(L.N[0] + 1 + kCgsOwnX - 1) / kCgsOwnX, (L.N[1] + kCgsOwnY - 1) / kCgsOwnY,
-                    (L.N[2] + kCgsPlanes - 1) / kCgsPlanes};
+    CgsTiles t{(L.N[0] + 1 + kCgsOwnX - 1) / kCgsOwnX, (L.N[1] + kCgsOwnY - 1) / kCgsOwnY, 0, 32};
+    do {
+        t.planes /= 2;
+        t.tz = (L.N[2] + t.planes - 1) / t.planes;
+    } while (t.planes > 2 && static_cast<long long>(t.tx) * t.ty * t.tz < kCgsFill);
+    return t;
+}
+
+// ---- one Jacobi diffusion iteration in one launch
+// Out of place, alternating between `out` and `in` as k_cgs_iter does:
+// src's iterate (with its ghosts) to dst on the fluid cells, the fill, and
+// the update norm.  Two things keep the reference's values
+// (JacobiDiffuse.cpp:85-99, :172-195): its `in` follows `out` on the domain
+// list only, so a fluid cell next to an obstacle always reads the obstacle
+// cell's entry value in `in`, whichever array holds the iterate; and those
+// cells of `in` are never written, so the fill's obstacle faces go to `out`
+// alone.  A ghost whose chain starts on an obstacle cell follows `out`.
+//
+// At 97x61x45 an iteration took five launches (sweep, two of fill, norm,
+// copy back; 18 us of kernels) and a readback that the host waited for;
+// so it takes two launches and four iterations are enqueued at once: 202 us
+// for a call of six iterations, 142 us so.
+// the update of fluid cell idx at (i, j, k), its coefficient rb and old value x
+template <bool TURB>
+__device__ __forceinline__ double jacobi_iter_update(const LevelDesc &L, const DiffCoef &c, double w, bool to_in,
+                                                     const double *__restrict__ src, const double *__restrict__ in,
+                                                     const double *__restrict__ b, const double *__restrict__ ev,
+                                                     int i, int j, int k, long long idx, double &rb, double &x) {
+    const long long nj = L.N[0], nk = static_cast<long long>(L.N[0]) * L.N[1];
+    double xp = src[idx + 1], xm = src[idx - 1], yp = src[idx + nj], ym = src[idx - nj], zp = src[idx + nk],
+           zm = src[idx - nk];
+    x = src[idx];
+    if (to_in) {
+        // one pass over the boxes: bit d set when neighbour d lies in one
+        unsigned solid = 0;
+        for (int o = 0; o < L.n_obst; o++) {
+            const int x0 = L.obst[o].lo[0], x1 = L.obst[o].hi[0], y0 = L.obst[o].lo[1], y1 = L.obst[o].hi[1],
+                      z0 = L.obst[o].lo[2], z1 = L.obst[o].hi[2];
+            const bool yz = j >= y0 && j <= y1 && k >= z0 && k <= z1, xz = i >= x0 && i <= x1 && k >= z0 && k <= z1,
+                       xy = i >= x0 && i <= x1 && j >= y0 && j <= y1;
+            solid |= (yz && i + 1 >= x0 && i + 1 <= x1 ? 1u : 0u) | (yz && i - 1 >= x0 && i - 1 <= x1 ? 2u : 0u) |
+                     (xz && j + 1 >= y0 && j + 1 <= y1 ? 4u : 0u) | (xz && j - 1 >= y0 && j - 1 <= y1 ? 8u : 0u) |
+                     (xy && k + 1 >= z0 && k + 1 <= z1 ? 16u : 0u) | (xy && k - 1 >= z0 && k - 1 <= z1 ? 32u : 0u);
+        }
+        if (solid) {
+            xp = solid & 1u ? in[idx + 1] : xp;
+            xm = solid & 2u ? in[idx - 1] : xm;
+            yp = solid & 4u ? in[idx + nj] : yp;
+            ym = solid & 8u ? in[idx - nj] : ym;
+            zp = solid & 16u ? in[idx + nk] : zp;
+            zm = solid & 32u ? in[idx - nk] : zm;
+        }
+    }
+    const double dsign = 1;
+    double out_h;
+    if (!TURB) {
+        rb = c.rb;
+        out_h = (dsign * b[idx] + c.ax * (xp + xm) + c.ay * (yp + ym) + c.az * (zp + zm)) / rb;
+    } else {
+        const double e = ev[idx];
+        const double aX = (c.D + e) * c.dt * c.rdx * c.rdx;
+        const double aY = (c.D + e) * c.dt * c.rdy * c.rdy;
+        const double aZ = (c.D + e) * c.dt * c.rdz * c.rdz;
+        rb = (1. + 2. * (aX + aY + aZ));
+        const double bb = 1. / rb;
+        out_h = bb * (dsign * b[idx] + aX * (xp + xm) + aY * (yp + ym) + aZ * (zp + zm));
+    }
+    return (1 - w) * x + w * out_h;
+}
+template <bool TURB>
+__global__ void k_jacobi_iter(LevelDesc L, BCView V, int main_z, int kz, DiffCoef c, double w,
+                              double *__restrict__ dst, const double *__restrict__ src, const double *__restrict__ in,
+                              const double *__restrict__ out, const double *__restrict__ b,
+                              const double *__restrict__ ev, double *__restrict__ partial, const int *gate) {
+    if (gate != nullptr && *gate) return;  // uniform over the grid
+    const bool to_in = src != in;          // (dst is `in`)
+    if (static_cast<int>(blockIdx.z) >= main_z) {
+        auto val = [&](long long q) -> double {
+            int i, j, k;
+            double rb, x;
+            if (!is_inner(L, q, i, j, k)) return out[q];
+            return jacobi_iter_update<TURB>(L, c, w, to_in, src, in, b, ev, i, j, k, q, rb, x);
+        };
+        const long long t = item_index(main_z);
+        if (to_in && t < V.n_faces) return;
+        dev::bc_item<double, decltype(val), true>(L, V, t, dst, val);
+        return;
+    }
+    int bx, by, bz;
+    main_block(main_z, bx, by, bz);
+    const int i = 1 + bx * BX + static_cast<int>(threadIdx.x);
+    const int j = 1 + by * BY + static_cast<int>(threadIdx.y);
+    double sq = 0.0;
+    if (i <= L.n[0] && j <= L.n[1])
+        for (int q = 0; q < kz; q++) {
+            const int k = 1 + bz * kz + q;
+            if (k > L.n[2]) break;
+            if (in_obstacle(L, i, j, k)) continue;
+            const long long idx = lin(L, i, j, k);
+            double rb, x;
+            const double v = jacobi_iter_update<TURB>(L, c, w, to_in, src, in, b, ev, i, j, k, idx, rb, x);
+            dst[idx] = v;
+            dev::face_ghosts(L, V, dst, idx, i, j, k, v);
+            const double r = rb * (v - x);
+            sq += r * r;
+        }
+    const double s = block_sum(sq);
+    if (threadIdx.x == 0 && threadIdx.y == 0)
+        partial[blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)] = s;
 }
 
 __global__ void k_swap(double *__restrict__ a, double *__restrict__ b, long long n) {
@@ -1112,8 +1224,14 @@ __global__ void k_fill_bc(LevelDesc L, BCView V, T *__restrict__ f) {
 // the fixed-order sum of k_reduce_sum, then the loop test of the diffusion
 // iteration (ColoredGaussSeidelDiffuse.cpp:60-98): run again while
 // sqrt(sum) > tol and fewer than max_iter iterations ran
-__global__ void k_reduce_gate(const double *__restrict__ partial, int n, IterGate *__restrict__ g) {
-    if (g->done) return;
+// (mirror: pinned host memory that receives the state, for the last
+// reduction before the host looks; a copy of it took a launch of its own)
+__global__ void k_reduce_gate(const double *__restrict__ partial, int n, IterGate *__restrict__ g,
+                              IterGate *__restrict__ mirror) {
+    if (g->done) {
+        if (mirror != nullptr && threadIdx.x == 0) *mirror = *g;
+        return;
+    }
     double v = 0.0;
     for (int t = threadIdx.x; t < n; t += 1024) v += partial[t];
     for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
@@ -1126,7 +1244,13 @@ __global__ void k_reduce_gate(const double *__restrict__ partial, int n, IterGat
         const int c = g->count + 1;
         g->sum = r;
         g->count = c;
-        g->done = (sqrt(r) > g->tol && c < g->max_iter) ? 0 : 1;
+        const int done = (sqrt(r) > g->tol && c < g->max_iter) ? 0 : 1;
+        g->done = done;
+        if (mirror != nullptr) {
+            mirror->sum = r;
+            mirror->count = c;
+            mirror->done = done;
+        }
     }
 }
 __global__ void k_log_gate(const IterGate *__restrict__ g, LoopLog *__restrict__ log) {
@@ -1353,12 +1477,28 @@ void cgs_iter(hipStream_t s, const LevelDesc &L, const BCView &V, const CgsCoef 
               const double *src, double *dst, double *partial, const int *gate) {
     const CgsTiles t = cgs_tiles(L);
     const long long main_blocks = static_cast<long long>(t.tx) * t.ty * t.tz;
-    const long long items = dev::bc_items_grid(V), per = 64 * kCgsWaves;
+    const long long items = dev::bc_items_grid(V) * kCgsItemLanes, per = 64 * kCgsWaves;
     const unsigned g = static_cast<unsigned>(main_blocks + (items + per - 1) / per);
     if (ev != nullptr)
         k_cgs_iter<true><<<g, dim3(64, kCgsWaves), 0, s>>>(L, V, t, c, ev, b, src, dst, partial, gate);
     else
         k_cgs_iter<false><<<g, dim3(64, kCgsWaves), 0, s>>>(L, V, t, c, ev, b, src, dst, partial, gate);
+}
+int jacobi_iter_partials(const LevelDesc &L, const BCView &V) {
+    const dim3 g = zbatch(inner_grid(L), kz_of(L, V));
+    return static_cast<int>(g.x * g.y * g.z);
+}
+void jacobi_iter(hipStream_t s, const LevelDesc &L, const BCView &V, double *dst, const double *src, const double *in,
+                 const double *out, const double *b, double ax, double ay, double az, double rb, double D,
+                 const double *ev, double dt, double w, double *partial, const int *gate) {
+    const DiffCoef c{ax, ay, az, rb, D, dt, 1. / L.h[0], 1. / L.h[1], 1. / L.h[2]};
+    const int kz = kz_of(L, V);
+    const dim3 g = zbatch(inner_grid(L), kz), gi = with_items(g, dev::bc_items_grid(V));
+    const int z = static_cast<int>(g.z);
+    if (ev != nullptr)
+        k_jacobi_iter<true><<<gi, block(), 0, s>>>(L, V, z, kz, c, w, dst, src, in, out, b, ev, partial, gate);
+    else
+        k_jacobi_iter<false><<<gi, block(), 0, s>>>(L, V, z, kz, c, w, dst, src, in, out, b, ev, partial, gate);
 }
 void swap_arrays(hipStream_t s, double *a, double *b, long long n) {
     k_swap<<<grid1d(n, 256), 256, 0, s>>>(a, b, n);
@@ -1533,8 +1673,8 @@ int partial_count(const LevelDesc &L) {
     const dim3 g = inner_grid(L);
     return static_cast<int>(g.x * g.y * g.z);
 }
-void reduce_gate(hipStream_t s, const double *partial, int n, IterGate *g) {
-    k_reduce_gate<<<1, 1024, 0, s>>>(partial, n, g);
+void reduce_gate(hipStream_t s, const double *partial, int n, IterGate *g, IterGate *mirror) {
+    k_reduce_gate<<<1, 1024, 0, s>>>(partial, n, g, mirror);
 }
 void gate_open(hipStream_t s, IterGate *g, double tol, int max_iter) { k_gate_open_iter<<<1, 64, 0, s>>>(g, tol, max_iter); }
 void log_gate(hipStream_t s, const IterGate *g, LoopLog *log) { k_log_gate<<<1, 64, 0, s>>>(g, log); }

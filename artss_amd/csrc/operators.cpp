@@ -67,6 +67,14 @@ void JacobiDiffuse::run(Field &out, const Field &in, const Field &b, double D, c
     StepCapture &cap = dm.capture();
     if (cap.mode == StepCapture::kCapture) throw capture_unsupported("the Jacobi diffusion loop");
     if (cap.mode == StepCapture::kRecord) cap.failed = true;
+    const int ft = out.get_type();
+    if (dm.bc_idempotent(0, ft)) {
+        const BCView V = dm.bc_view(0, ft);
+        if (k::jacobi_iter_partials(L, V) <= dm.partial_capacity()) {
+            run_one_pass(out, in, b, D, EV ? EV->data : nullptr, V);
+            return;
+        }
+    }
     int it = 0;
     double res = 1.;
     while (res > m_settings.tol_res && it < m_settings.max_iter) {
@@ -82,6 +90,50 @@ void JacobiDiffuse::run(Field &out, const Field &in, const Field &b, double D, c
     if (it % 2 != 0) k::copy_domain(dm.stream(), L, in.data, out.data);
     m_iterations = it;
     m_residual = res;
+}
+
+// The same loop with each iteration as one out-of-place launch
+// (k::jacobi_iter), alternating between the two arrays.  After an odd count
+// `out` holds the last iterate with its fill and `in` follows it on the
+// domain list; after an even count the iterate stands in `in`, `out` takes it
+// over and its obstacle faces are filled.
+void JacobiDiffuse::run_one_pass(Field &out, const Field &in, const Field &b, double D, const double *ev,
+                                 const BCView &V) {
+    Domain &dm = m_domain;
+    const LevelDesc &L = dm.level(0);
+    hipStream_t s = dm.stream();
+    const double dt = dm.settings().dt;
+    const double rdx = 1. / L.h[0], rdy = 1. / L.h[1], rdz = 1. / L.h[2];
+    const double ax = D * dt * rdx * rdx, ay = D * dt * rdy * rdy, az = D * dt * rdz * rdz;
+    const double rb = (1. + 2. * (ax + ay + az));
+    k::IterGate *gate = dm.loop_gate(), *mirror = dm.loop_mirror();
+    const int *stop = &gate->done;
+    const int n_part = k::jacobi_iter_partials(L, V);
+    k::gate_open(s, gate, m_settings.tol_res, m_settings.max_iter);
+    int launched = 0;
+    do {
+        const int n = batch(launched);
+        for (int q = 0; q < n; q++) {
+            const bool odd = ((launched + q) & 1) == 0;  // iteration number launched + q + 1
+            dm.timed("jacobi_diffuse", 0, [&] {
+                k::jacobi_iter(s, L, V, odd ? out.data : in.data, odd ? in.data : out.data, in.data, out.data, b.data,
+                               ax, ay, az, rb, D, ev, dt, m_settings.w, dm.partial_buffer(), stop);
+            });
+            k::reduce_gate(s, dm.partial_buffer(), n_part, gate, q + 1 == n ? mirror : nullptr);
+        }
+        launched += n;
+        ARTSS_HIP(hipStreamSynchronize(s));
+    } while (!mirror->done);
+    m_iterations = mirror->count;
+    m_residual = m_iterations > 0 ? std::sqrt(mirror->sum) : 1.;
+    m_hint = m_iterations;
+    if (m_iterations == 0) return;
+    if (m_iterations % 2 != 0) {
+        k::copy_domain(s, L, in.data, out.data);
+    } else {
+        k::copy_domain(s, L, out.data, in.data);
+        dm.apply_faces(out.data, out.get_type(), 0);
+    }
 }
 
 void JacobiDiffuse::diffuse(Field &out, const Field &in, const Field &b, double D, bool sync) {
@@ -124,16 +176,12 @@ void ColoredGaussSeidelDiffuse::run(Field &out, const Field &in, const Field &b,
     const double rb = (1. + 2. * (ax + ay + az));
     const double beta = 1. / rb;
     const double *ev = EV ? EV->data : nullptr;
-    // The loop test runs on the device (k::IterGate): as many iterations as
-    // the previous call took are enqueued at once, then one at a time; the
-    // kernels of iterations past the test's stop do nothing, so the fields
-    // are those of the reference's loop, which tests after every iteration.
+    // The loop test runs on the device (GatedLoop): the kernels of iterations
+    // past the test's stop do nothing, so the fields are those of the
+    // reference's loop, which tests after every iteration.
     hipStream_t s = dm.stream();
-    if (!m_gate) {
-        ARTSS_HIP(hipMalloc(&m_gate, sizeof(k::IterGate)));
-        ARTSS_HIP(hipHostMalloc(&m_gate_host, sizeof(k::IterGate)));
-    }
-    const int *stop = &m_gate->done;
+    k::IterGate *gate = dm.loop_gate(), *mirror = dm.loop_mirror();
+    const int *stop = &gate->done;
     const int ft = out.get_type();
     if (dm.bc_idempotent(0, ft)) {
         const BCView V = dm.bc_view(0, ft);
@@ -149,11 +197,11 @@ void ColoredGaussSeidelDiffuse::run(Field &out, const Field &in, const Field &b,
     if (cap.mode == StepCapture::kRecord) cap.failed = true;
     const int n_part = k::partial_count(L);
     out.copy_data(in);
-    k::gate_open(s, m_gate, m_settings.tol_res, m_settings.max_iter);
+    k::gate_open(s, gate, m_settings.tol_res, m_settings.max_iter);
     int launched = 0;
-    while (true) {
-        const int batch = launched < m_batch_hint ? m_batch_hint - launched : 1;
-        for (int q = 0; q < batch; q++) {
+    do {
+        const int n = batch(launched);
+        for (int q = 0; q < n; q++) {
             k::copy(s, in.data, out.data, in.get_size(), stop);
             for (int color = 0; color < 2; color++)
                 dm.timed("cgs_diffuse", 0, [&] {
@@ -162,16 +210,14 @@ void ColoredGaussSeidelDiffuse::run(Field &out, const Field &in, const Field &b,
                 });
             dm.apply_boundary(out.data, out.get_type(), 0, stop);
             k::update_norm_partials(s, L, out.data, in.data, rb, D, ev, dt, dm.partial_buffer(), stop);
-            k::reduce_gate(s, dm.partial_buffer(), n_part, m_gate);
+            k::reduce_gate(s, dm.partial_buffer(), n_part, gate, q + 1 == n ? mirror : nullptr);
         }
-        launched += batch;
-        ARTSS_HIP(hipMemcpyAsync(m_gate_host, m_gate, sizeof(k::IterGate), hipMemcpyDeviceToHost, s));
+        launched += n;
         ARTSS_HIP(hipStreamSynchronize(s));
-        if (m_gate_host->done) break;
-    }
-    m_iterations = m_gate_host->count;
-    m_residual = m_iterations > 0 ? std::sqrt(m_gate_host->sum) : 1.;
-    m_batch_hint = m_iterations;
+    } while (!mirror->done);
+    m_iterations = mirror->count;
+    m_residual = m_iterations > 0 ? std::sqrt(mirror->sum) : 1.;
+    m_hint = m_iterations;
 }
 
 // The same loop with each iteration as one out-of-place kernel
@@ -187,9 +233,10 @@ void ColoredGaussSeidelDiffuse::run_one_pass(Field &out, const Field &in, const 
     Domain &dm = m_domain;
     const LevelDesc &L = dm.level(0);
     hipStream_t s = dm.stream();
-    const int *stop = &m_gate->done;
+    k::IterGate *gate = dm.loop_gate(), *mirror = dm.loop_mirror();
+    const int *stop = &gate->done;
     const int n_part = k::cgs_iter_partials(L);
-    k::gate_open(s, m_gate, m_settings.tol_res, m_settings.max_iter);
+    k::gate_open(s, gate, m_settings.tol_res, m_settings.max_iter);
     StepCapture &cap = dm.capture();
     if (cap.mode == StepCapture::kCapture) {
         // a fixed budget behind the gate; the arrays' final exchange and the
@@ -201,45 +248,35 @@ void ColoredGaussSeidelDiffuse::run_one_pass(Field &out, const Field &in, const 
             const bool odd = (q & 1) == 0;
             k::cgs_iter(s, L, V, c, ev, b.data, odd ? in.data : out.data, odd ? out.data : in.data,
                         dm.partial_buffer(), stop);
-            k::reduce_gate(s, dm.partial_buffer(), n_part, m_gate);
+            k::reduce_gate(s, dm.partial_buffer(), n_part, gate);
         }
-        k::alternate_finish(s, m_gate, out.data, in.data, out.get_size());
-        k::log_gate(s, m_gate, cap.log + slot);
+        k::alternate_finish(s, gate, out.data, in.data, out.get_size());
+        k::log_gate(s, gate, cap.log + slot);
         return;
     }
     int launched = 0;
-    while (true) {
-        const int batch = launched < m_batch_hint ? m_batch_hint - launched : 1;
-        for (int q = 0; q < batch; q++) {
+    do {
+        const int n = batch(launched);
+        for (int q = 0; q < n; q++) {
             const bool odd = ((launched + q) & 1) == 0;  // iteration number launched + q + 1
             const double *src = odd ? in.data : out.data;
             double *dst = odd ? out.data : in.data;
             dm.timed("cgs_diffuse", 0, [&] {
                 k::cgs_iter(s, L, V, c, ev, b.data, src, dst, dm.partial_buffer(), stop);
             });
-            k::reduce_gate(s, dm.partial_buffer(), n_part, m_gate);
+            k::reduce_gate(s, dm.partial_buffer(), n_part, gate, q + 1 == n ? mirror : nullptr);
         }
-        launched += batch;
-        ARTSS_HIP(hipMemcpyAsync(m_gate_host, m_gate, sizeof(k::IterGate), hipMemcpyDeviceToHost, s));
+        launched += n;
         ARTSS_HIP(hipStreamSynchronize(s));
-        if (m_gate_host->done) break;
-    }
-    m_iterations = m_gate_host->count;
-    m_residual = m_iterations > 0 ? std::sqrt(m_gate_host->sum) : 1.;
-    m_batch_hint = m_iterations;
+    } while (!mirror->done);
+    m_iterations = mirror->count;
+    m_residual = m_iterations > 0 ? std::sqrt(mirror->sum) : 1.;
+    m_hint = m_iterations;
     if (m_iterations == 0) out.copy_data(in);
     else if (m_iterations % 2 == 0) k::swap_arrays(s, out.data, in.data, out.get_size());
     if (cap.mode == StepCapture::kRecord) {
         cap.counts.push_back(m_iterations);
         cap.kinds.push_back(StepCapture::kDiffusion);
-    }
-}
-
-ColoredGaussSeidelDiffuse::~ColoredGaussSeidelDiffuse() {
-    if (m_gate) {
-        (void)hipStreamSynchronize(m_domain.stream());
-        (void)hipFree(m_gate);
-        (void)hipHostFree(m_gate_host);
     }
 }
 

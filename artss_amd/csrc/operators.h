@@ -85,8 +85,20 @@ class SLAdvect : public IAdvection {
     Domain &m_domain;
 };
 
+// The residual-target loops test on the device (k::IterGate): several
+// iterations are enqueued before the host looks at the state, and those past
+// the test's stop do nothing.  An object that ran before enqueues its last
+// count at once; a new one four (a gated launch costs 2 to 5 us, a look about
+// 15 us of idle device), then more in fours or one by one.
+class GatedLoop {
+  protected:
+    // iterations to enqueue when `launched` have been
+    int batch(int launched) const { return launched < m_hint ? m_hint - launched : (m_hint > 0 ? 1 : 4); }
+    int m_hint = 0;  // iterations of the previous call
+};
+
 // diffusion/JacobiDiffuse.cpp:31-203
-class JacobiDiffuse : public IDiffusion {
+class JacobiDiffuse : public IDiffusion, private GatedLoop {
   public:
     JacobiDiffuse(Domain &d, const DiffusionSettings &s) : m_domain(d), m_settings(s) {}
     void diffuse(Field &out, const Field &in, const Field &b, double D, bool sync) override;
@@ -94,6 +106,7 @@ class JacobiDiffuse : public IDiffusion {
 
   private:
     void run(Field &out, const Field &in, const Field &b, double D, const Field *EV);
+    void run_one_pass(Field &out, const Field &in, const Field &b, double D, const double *ev, const BCView &V);
     Domain &m_domain;
     DiffusionSettings m_settings;
 };
@@ -111,12 +124,9 @@ class ExplicitDiffuse : public IDiffusion {
 };
 
 // diffusion/ColoredGaussSeidelDiffuse.cpp:38-173
-class ColoredGaussSeidelDiffuse : public IDiffusion {
+class ColoredGaussSeidelDiffuse : public IDiffusion, private GatedLoop {
   public:
     ColoredGaussSeidelDiffuse(Domain &d, const DiffusionSettings &s) : m_domain(d), m_settings(s) {}
-    ~ColoredGaussSeidelDiffuse() override;
-    ColoredGaussSeidelDiffuse(const ColoredGaussSeidelDiffuse &) = delete;
-    ColoredGaussSeidelDiffuse &operator=(const ColoredGaussSeidelDiffuse &) = delete;
     void diffuse(Field &out, const Field &in, const Field &b, double D, bool sync) override;
     void diffuse(Field &out, const Field &in, const Field &b, double D, const Field &EV, bool sync) override;
 
@@ -126,9 +136,6 @@ class ColoredGaussSeidelDiffuse : public IDiffusion {
                       const k::CgsCoef &c);
     Domain &m_domain;
     DiffusionSettings m_settings;
-    k::IterGate *m_gate = nullptr;       // device loop state
-    k::IterGate *m_gate_host = nullptr;  // pinned
-    int m_batch_hint = 0;                // iterations of the previous call, enqueued at once
 };
 
 // turbulence/ConstSmagorinsky.cpp:30-97
