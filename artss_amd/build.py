@@ -17,7 +17,7 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libartss_hip.so")
 ARCH = os.environ.get("ARTSS_OFFLOAD_ARCH", "gfx950")
 
-SOURCES = ["kernels.hip", "mg_tail.hip", "krylov_kernels.hip", "krylov.cpp", "unet_kernels.hip", "unet.cpp",
+SOURCES = ["kernels.hip", "mg_tail.hip", "mg_fused.hip", "krylov_kernels.hip", "krylov.cpp", "unet_kernels.hip", "unet.cpp",
            "domain.cpp", "operators.cpp", "dyn_smagorinsky.cpp", "vcycle.cpp", "solver.cpp", "functions.cpp", "ensemble.cpp", "settings.cpp", "xml.cpp",
            "residual_static.hip", "capi.cpp"]
 

@@ -95,9 +95,29 @@ struct BCView {
     const uint32_t *rest;
     long long n_rest;
     // every ghost cell is written by the fill: kernels that must write every
-    // cell (first sweeps, the out-of-place prolongation, copy_bc) can then
+    // cell (first sweeps, the out-of-place prolongation) can then
     // run over the inner box only
     int shell_filled;
+};
+
+// An idempotent fill of zero values, resolved cell by cell (mg_fused.hip)
+struct MgFill {
+    // per cell of the level, ghosts included: n + 1 for a fluid cell n;
+    // source + 1, or -(source + 1) where the signs multiply to -1, for a cell
+    // the fill sets from `source` (a cell it does not write); else 0
+    const int32_t *src_of;
+    // the cells a sweep's own thread does not write: obstacle faces, edges,
+    // corners and ghosts of obstacle faces, and the shell cells the fill
+    // leaves alone.  Eight words each: s + 1 of the cell s whose value the
+    // item takes (negative: s is not fluid, it keeps the iterate's value),
+    // src_of of its neighbours x + 1, x - 1, y + 1, y - 1, z + 1, z - 1, and
+    // the cell written + 1 (negative: with sign -1)
+    const int32_t *items;
+    int n_items;
+    // face ghosts set from an inner fluid cell: target coordinate and sign
+    int active;
+    int target[6];
+    double sign[6];
 };
 
 #if defined(__HIPCC__)

@@ -152,6 +152,7 @@ Domain::~Domain() {
     (void)hipFree(m_params_dev);
     (void)hipFree(m_params_hom_dev);
     (void)hipFree(m_bits_dev);
+    (void)hipFree(m_mg_dev);
     (void)hipFree(m_deps_dev);
     (void)hipFree(m_rest_dev);
     (void)hipStreamDestroy(m_stream);
@@ -326,6 +327,8 @@ void Domain::build_boundary_tables() {
     std::vector<uint32_t> bits;
     std::vector<DepGhost> deps;
     std::vector<uint32_t> rest;
+    std::vector<int32_t> mg;
+    m_mg_table.assign(m_levels + 1, MgTable());
     m_idem.assign(m_levels + 1, std::vector<char>(NUMBER_OF_FIELD_TYPES, 0));
     m_face_values_zero.assign(m_levels + 1, std::vector<char>(NUMBER_OF_FIELD_TYPES, 1));
     m_view_bits.assign(m_levels + 1, std::vector<long long>(NUMBER_OF_FIELD_TYPES, 0));
@@ -570,6 +573,65 @@ void Domain::build_boundary_tables() {
                     rest.push_back(static_cast<uint32_t>(g));
                 }
                 m_view_nrest[l][f] = static_cast<long long>(rest.size()) - m_view_rest[l][f];
+                if (f == P && m_levels > 0) {
+                    MgTable &M = m_mg_table[l];
+                    M.map = static_cast<long long>(mg.size());
+                    mg.resize(mg.size() + static_cast<size_t>(L.size), 0);
+                    int32_t *map = &mg[static_cast<size_t>(M.map)];
+                    for (int k = 1; k <= L.n[2]; k++)
+                        for (int j = 1; j <= L.n[1]; j++)
+                            for (int i = 1; i <= L.n[0]; i++)
+                                if (!in_obstacle(L, i, j, k)) {
+                                    const long long c = i + Nx * (j + Ny * static_cast<long long>(k));
+                                    map[c] = static_cast<int32_t>(c + 1);
+                                }
+                    std::vector<long long> own;  // cells written by items
+                    const Wave W0 = m_waves[l][f].empty() ? Wave{0, 0} : m_waves[l][f][0];
+                    for (long long e = W0.offset; e < W0.offset + W0.count; e++) {
+                        const FaceEntry &x = entries[static_cast<size_t>(e)];
+                        const long long src = static_cast<long long>(x.idx) + x.ref;
+                        const bool neg = params[static_cast<size_t>(m_param_offset[l][f] + x.param)].sign < 0.0;
+                        map[x.idx] = static_cast<int32_t>(neg ? -(src + 1) : src + 1);
+                        if (written[x.idx] == 2) own.push_back(x.idx);
+                    }
+                    for (size_t t0 = 0; t0 < ghost_src.size(); t0++) {
+                        const long long g = ghost_cell[t0];
+                        const long long i = g % Nx, j = (g / Nx) % Ny, k = g / (Nx * Ny);
+                        double sign = 1.0;
+                        if (i == 0 || i == Nx - 1) sign *= d.sign[i == 0 ? 0 : 1];
+                        if (j == 0 || j == Ny - 1) sign *= d.sign[j == 0 ? 2 : 3];
+                        if (k == 0 || k == Nz - 1) sign *= d.sign[k == 0 ? 4 : 5];
+                        // (the source is a cell the fill does not write or an obstacle face)
+                        const long long src = ghost_src[t0];
+                        const int32_t e = written[static_cast<size_t>(src)] ? map[src] : static_cast<int32_t>(src + 1);
+                        map[g] = sign < 0.0 ? -e : e;
+                    }
+                    for (long long q = m_view_deps[l][f]; q < m_view_deps[l][f] + m_view_ndeps[l][f]; q++)
+                        own.push_back(deps[static_cast<size_t>(q)].idx);
+                    for (long long q = m_view_rest[l][f]; q < m_view_rest[l][f] + m_view_nrest[l][f]; q++)
+                        own.push_back(rest[static_cast<size_t>(q)]);
+                    if (!shell)
+                        for (long long c = 0; c < L.size; c++) {
+                            const long long i = c % Nx, j = (c / Nx) % Ny, k = c / (Nx * Ny);
+                            if ((i == 0 || j == 0 || k == 0 || i == Nx - 1 || j == Ny - 1 || k == Nz - 1) &&
+                                !written[static_cast<size_t>(c)])
+                                own.push_back(c);
+                        }
+                    M.n_items = static_cast<int>(own.size());
+                    std::vector<int32_t> items(8 * own.size(), 0);
+                    const long long off[6] = {1, -1, Nx, -Nx, Nx * Ny, -Nx * Ny};
+                    for (size_t q = 0; q < own.size(); q++) {
+                        const long long c = own[q];
+                        const int32_t e = map[c];
+                        const long long src = e == 0 ? c : (e < 0 ? -e : e) - 1;
+                        const bool fluid = map[src] == static_cast<int32_t>(src + 1);
+                        items[8 * q] = static_cast<int32_t>(fluid ? src + 1 : -(src + 1));
+                        for (int a = 0; a < 6 && fluid; a++) items[8 * q + 1 + a] = map[src + off[a]];
+                        items[8 * q + 7] = static_cast<int32_t>(e < 0 ? -(c + 1) : c + 1);
+                    }
+                    M.items = static_cast<long long>(mg.size());
+                    mg.insert(mg.end(), items.begin(), items.end());
+                }
             }
         }
     }
@@ -591,6 +653,10 @@ void Domain::build_boundary_tables() {
     if (!bits.empty()) {
         ARTSS_HIP(hipMalloc(&m_bits_dev, sizeof(uint32_t) * bits.size()));
         ARTSS_HIP(hipMemcpy(m_bits_dev, bits.data(), sizeof(uint32_t) * bits.size(), hipMemcpyHostToDevice));
+    }
+    if (!mg.empty()) {
+        ARTSS_HIP(hipMalloc(&m_mg_dev, sizeof(int32_t) * mg.size()));
+        ARTSS_HIP(hipMemcpy(m_mg_dev, mg.data(), sizeof(int32_t) * mg.size(), hipMemcpyHostToDevice));
     }
     if (!deps.empty()) {
         ARTSS_HIP(hipMalloc(&m_deps_dev, sizeof(DepGhost) * deps.size()));
@@ -621,6 +687,22 @@ BCView Domain::bc_view(int level, int ft, bool homogeneous) const {
     v.n_ghosts = v.bc.active ? ghost_cells(level) : 0;
     v.shell_filled = m_shell[level][ft];
     return v;
+}
+
+MgFill Domain::mg_fill(int level) const {
+    const MgTable &M = m_mg_table[static_cast<size_t>(level)];
+    if (M.map < 0 || m_mg_dev == nullptr) throw std::logic_error("mg_fill of a level without an idempotent fill");
+    MgFill f{};
+    f.src_of = m_mg_dev + M.map;
+    f.items = m_mg_dev + M.items;
+    f.n_items = M.n_items;
+    const DomainBC &d = m_dom_bc[level][P];
+    f.active = d.active;
+    for (int p = 0; p < 6; p++) {
+        f.target[p] = d.target[p];
+        f.sign[p] = d.sign[p];
+    }
+    return f;
 }
 
 bool Domain::bc_values_zero(int level, int ft) const {

@@ -93,6 +93,9 @@ class Domain {
     // then produce the filled values themselves from bc_view.
     bool bc_idempotent(int level, int field_type) const { return m_idem[level][field_type] != 0; }
     // homogeneous: the same fill with every boundary value zero (its linear part)
+    // the pressure-type fill of a multigrid level whose fill is idempotent,
+    // with every value taken as zero
+    MgFill mg_fill(int level) const;
     BCView bc_view(int level, int field_type, bool homogeneous = false) const;
     // the fill has no non-zero boundary value (it is linear)
     bool bc_values_zero(int level, int field_type) const;
@@ -197,6 +200,12 @@ class Domain {
     std::vector<std::vector<long long>> m_view_bits, m_view_deps, m_view_ndeps, m_view_rest, m_view_nrest;
     uint32_t *m_rest_dev = nullptr;
     uint32_t *m_bits_dev = nullptr;
+    int32_t *m_mg_dev = nullptr;  // MgFill tables of the pressure-type fills, per level the map, then the items
+    struct MgTable {
+        long long map = -1, items = 0;  // offsets (-1: none)
+        int n_items = 0;
+    };
+    std::vector<MgTable> m_mg_table;
     DepGhost *m_deps_dev = nullptr;
     long long m_face_entries = 0;
     FaceEntry *m_faces_dev = nullptr;

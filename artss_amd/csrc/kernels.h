@@ -15,9 +15,11 @@ namespace k {
 // gate (optional): nothing runs while *gate != 0 (IterGate::done)
 void copy(hipStream_t s, double *dst, const double *src, long long n, const int *gate = nullptr);
 // x[cells[r]] = sum_j M[r * n + j] b[cells[j]] for r < n (n <= kMaxDenseRows:
-// the gathered b is staged in 16 KiB of LDS per workgroup)
+// the gathered b is staged in 16 KiB of LDS per workgroup), and the fill of
+// zero values: cell |d| - 1 takes +-x[cells[r]] for d in deps[ptr[r] .. ptr[r + 1])
 constexpr int kMaxDenseRows = 2048;
-void dense_apply(hipStream_t s, int n, const double *M, const uint32_t *cells, const double *b, double *x);
+void dense_apply(hipStream_t s, int n, const double *M, const uint32_t *cells, const uint32_t *ptr,
+                 const int32_t *deps, const double *b, double *x);
 // dst0[q] = dst1[q] = src[q] for q < fields (1..4), n elements each, one pass
 struct CopyFan {
     const double *src[4];
@@ -116,11 +118,6 @@ void prolongate_add(hipStream_t s, const LevelDesc &Lc, const LevelDesc &Lf, dou
 // Iterates of type T (double: the reference's arithmetic; float: the mixed
 // V-cycle), right-hand sides / coarse errors of type TB / Tc.
 void copy_bc(hipStream_t s, const LevelDesc &L, const BCView &V, double *dst, const double *src);
-// restrict_fill<float, float, float> into rhs followed by the coarse level's
-// first sweep from zero into err with its fill (jacobi_bc with src == nullptr),
-// in one launch; the values are those of the two launches
-void restrict_sweep0(hipStream_t s, const LevelDesc &Lc, const LevelDesc &Lf, const BCView &V, float *rhs, float *err,
-                     const float *fine, double ax, double ay, double az, double beta, double dsign, double w);
 // autotuner of the fused level kernels' cells per thread along z (1, 2 or 4)
 // for a level size, timed on scratch arrays; call outside stream capture
 void tune_level(hipStream_t s, const LevelDesc &L, const BCView &V);

@@ -1164,54 +1164,47 @@ __global__ void k_prolongate_add_bc(LevelDesc Lc, LevelDesc Lf, BCView V, int ma
 }
 
 // x[cells[r]] = sum_j M[r][j] b[cells[j]]: one wavefront per row, the
-// gathered right-hand side staged in LDS, a fixed summation order
+// gathered right-hand side staged in LDS, a fixed summation order.  The cells
+// the fill sets from cells[r] follow in deps[ptr[r] .. ptr[r + 1]) (cell + 1,
+// negative: with sign -1).  Bound by latency (the matrix of 1012 rows takes
+// 2 us to read): a lane's first eight entries are on their way while the
+// right-hand side is staged, and the fill needs no launch of its own (9 + 5
+// us before).
 __global__ void k_dense_apply(int n, const double *__restrict__ M, const uint32_t *__restrict__ cells,
+                              const uint32_t *__restrict__ ptr, const int32_t *__restrict__ deps,
                               const double *__restrict__ b, double *__restrict__ x) {
     extern __shared__ double sb[];
-    for (int j = static_cast<int>(threadIdx.x); j < n; j += static_cast<int>(blockDim.x)) sb[j] = b[cells[j]];
-    __syncthreads();
     const int lane = static_cast<int>(threadIdx.x) & 63;
     const int row = static_cast<int>(blockIdx.x) * (static_cast<int>(blockDim.x) >> 6) +
                     (static_cast<int>(threadIdx.x) >> 6);
+    const double *m = M + static_cast<size_t>(row < n ? row : 0) * static_cast<size_t>(n);
+    constexpr int kChunk = 8;
+    double a[kChunk];
+#pragma unroll
+    for (int q = 0; q < kChunk; q++) a[q] = lane + 64 * q < n ? m[lane + 64 * q] : 0.0;
+    for (int j = static_cast<int>(threadIdx.x); j < n; j += static_cast<int>(blockDim.x)) sb[j] = b[cells[j]];
+    __syncthreads();
     if (row >= n) return;
-    const double *m = M + static_cast<size_t>(row) * static_cast<size_t>(n);
     double acc = 0.0;
-    for (int j = lane; j < n; j += 64) acc += m[j] * sb[j];
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-    if (lane == 0) x[cells[row]] = acc;
-}
-
-// Restriction of the fine residuum to a coarse level fused with that level's
-// first smoothing sweep from zero (k_restrict_fill, then k_jacobi_bc with
-// ZERO): rhs = restrict(fine) on the coarse fluid cells, err = w beta dsign
-// rhs there, err's fill, zero on every other cell.  Fill items restrict the
-// cell they read themselves, so no cell waits for another workgroup.
-__global__ void k_restrict_sweep0(LevelDesc Lc, LevelDesc Lf, BCView V, int main_z, float w, float beta, float dsign,
-                                  float *__restrict__ rhs, float *__restrict__ err, const float *__restrict__ fine) {
-    if (static_cast<int>(blockIdx.z) >= main_z) {
-        auto val = [&](long long c) -> float {
-            int ci, cj, ck;
-            if (!is_inner(Lc, c, ci, cj, ck)) return 0.0f;
-            return w * (beta * (dsign * dev::restrict_t<float>(Lf, fine, ci, cj, ck)));
-        };
-        dev::bc_item<float, decltype(val), true>(Lc, V, item_index(main_z), err, val);
-        return;
+    for (int j0 = lane; j0 < n; j0 += 64 * kChunk) {
+        double next[kChunk];
+#pragma unroll
+        for (int q = 0; q < kChunk; q++) {
+            const int j = j0 + 64 * (kChunk + q);
+            next[q] = j < n ? m[j] : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < kChunk; q++)
+            if (j0 + 64 * q < n) acc += a[q] * sb[j0 + 64 * q];
+#pragma unroll
+        for (int q = 0; q < kChunk; q++) a[q] = next[q];
     }
-    int bx, by, bz;
-    main_block(main_z, bx, by, bz);
-    const int i = bx * BX + static_cast<int>(threadIdx.x);
-    const int j = by * BY + static_cast<int>(threadIdx.y);
-    const int k = bz;
-    if (i >= Lc.N[0] || j >= Lc.N[1]) return;
-    const long long idx = lin(Lc, i, j, k);
-    if (i >= 1 && j >= 1 && k >= 1 && i <= Lc.n[0] && j <= Lc.n[1] && k <= Lc.n[2] && !in_obstacle(Lc, i, j, k)) {
-        const float r = dev::restrict_t<float>(Lf, fine, i, j, k);
-        rhs[idx] = r;
-        const float v = w * (beta * (dsign * r));
-        err[idx] = v;
-        dev::face_ghosts(Lc, V, err, idx, i, j, k, v);
-    } else if (!dev::written(V, idx)) {
-        err[idx] = 0.0f;
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+    acc = __shfl(acc, 0, 64);
+    if (lane == 0) x[cells[row]] = acc;
+    for (uint32_t q = ptr[row] + static_cast<uint32_t>(lane); q < ptr[row + 1]; q += 64) {
+        const int32_t d = deps[q];
+        x[(d < 0 ? -d : d) - 1] = (d < 0 ? -1.0 : 1.0) * acc + 0.0;
     }
 }
 
@@ -1378,9 +1371,10 @@ __global__ void k_buoyancy(LevelDesc L, double beta, double g, double *__restric
 void copy(hipStream_t s, double *dst, const double *src, long long n, const int *gate) {
     k_copy<<<grid1d(n, 256), 256, 0, s>>>(dst, src, n, gate);
 }
-void dense_apply(hipStream_t s, int n, const double *M, const uint32_t *cells, const double *b, double *x) {
+void dense_apply(hipStream_t s, int n, const double *M, const uint32_t *cells, const uint32_t *ptr,
+                 const int32_t *deps, const double *b, double *x) {
     if (n < 1 || n > kMaxDenseRows) throw std::invalid_argument("dense_apply: 1 to kMaxDenseRows rows");
-    k_dense_apply<<<(n + 3) / 4, 256, sizeof(double) * static_cast<size_t>(n), s>>>(n, M, cells, b, x);
+    k_dense_apply<<<(n + 3) / 4, 256, sizeof(double) * static_cast<size_t>(n), s>>>(n, M, cells, ptr, deps, b, x);
 }
 void copy_fan(hipStream_t s, const CopyFan &f, long long n) {
     switch (f.fields) {
@@ -1527,16 +1521,6 @@ template void restrict_fill<float, float, float>(hipStream_t, const LevelDesc &,
                                                  const float *, float *);
 template void restrict_fill<float, double, double>(hipStream_t, const LevelDesc &, const LevelDesc &, double *,
                                                    const float *, double *);
-void restrict_sweep0(hipStream_t s, const LevelDesc &Lc, const LevelDesc &Lf, const BCView &V, float *rhs, float *err,
-                     const float *fine, double ax, double ay, double az, double beta, double dsign, double w) {
-    (void)ax;
-    (void)ay;
-    (void)az;
-    const dim3 g = full_grid(Lc);
-    k_restrict_sweep0<<<with_items(g, dev::bc_items_grid(V)), block(), 0, s>>>(
-        Lc, Lf, V, static_cast<int>(g.z), static_cast<float>(w), static_cast<float>(beta), static_cast<float>(dsign), rhs,
-        err, fine);
-}
 void prolongate_add(hipStream_t s, const LevelDesc &Lc, const LevelDesc &Lf, double *fine, const double *coarse) {
     k_prolongate_add<<<inner_grid(Lc), block(), 0, s>>>(Lc, Lf, fine, coarse);
 }
@@ -1655,10 +1639,6 @@ void prolongate_add_bc(hipStream_t s, const LevelDesc &Lc, const LevelDesc &Lf, 
 }
 template void prolongate_add_bc<double, double>(hipStream_t, const LevelDesc &, const LevelDesc &, const BCView &,
                                                 double *, const double *, const double *);
-template void prolongate_add_bc<float, double>(hipStream_t, const LevelDesc &, const LevelDesc &, const BCView &,
-                                               float *, const float *, const double *);
-template void prolongate_add_bc<float, float>(hipStream_t, const LevelDesc &, const LevelDesc &, const BCView &,
-                                              float *, const float *, const float *);
 
 template <typename T>
 void fill_bc(hipStream_t s, const LevelDesc &L, const BCView &V, T *f) {

@@ -47,11 +47,12 @@ bool VCycleMG::mixed_supported() const {
 }
 
 void VCycleMG::free_mixed() {
-    for (auto *v : {&m_err1f, &m_tmpf, &m_scrf, &m_res0f, &m_res1f}) {
+    for (auto *v : {&m_err1f, &m_tmpf, &m_res0f, &m_res1f}) {
         for (float *p : *v)
             if (p) (void)hipFree(p);
         v->clear();
     }
+    m_mixed_out = nullptr;
 }
 
 void VCycleMG::alloc_mixed() {
@@ -69,60 +70,50 @@ void VCycleMG::alloc_mixed() {
     for (int l = 0; l < f; l++) {
         m_err1f.push_back(alloc(l));
         m_tmpf.push_back(alloc(l));
-        m_scrf.push_back(alloc(l));
-        m_res0f.push_back(alloc(l));
+        m_res0f.push_back(restrict_reads_ghost(l) ? alloc(l) : nullptr);
         m_res1f.push_back(l > 0 ? alloc(l) : nullptr);
     }
 }
 
-// smooth_fast in FP32: tmpf -> err1f -> ... -> err1f, linear part of the fill
-// `sweeps` weighted-Jacobi sweeps from tmp into err1 (0: the XML's
-// effective count).  An even count starts with one sweep into a third
-// buffer, so the result always lands in err1; the first sweep into a buffer
-// copies the cells it does not update, so err1 holds tmp's values there.
+// effective sweeps for a count (0: the XML's)
 int VCycleMG::mixed_sweep_count(int sweeps) const {
     const int nx = m_s.n_relax;
     return sweeps > 0 ? sweeps : ((nx % 2 == 0 && nx > 0) ? nx - 1 : nx);
 }
 
-float *VCycleMG::first_sweep_target(int level, int sweeps) const {
-    const int n = mixed_sweep_count(sweeps);
-    return (n % 2 == 0 && n > 0) ? m_scrf[level] : m_err1f[level];
+k::MgSweep VCycleMG::mixed_sweep(int level) const {
+    k::MgSweep c{};
+    coeffs(level, &c.ax, &c.ay, &c.az, &c.beta);
+    c.dsign = kDsign;
+    c.w = m_mixed_weight > 0.0 ? m_mixed_weight : m_s.smoother.w;
+    return c;
 }
 
-void VCycleMG::smooth_fast_f(int level, const double *b64, const float *b32, int sweeps, bool from_zero,
-                             bool first_done) {
+// `sweeps` weighted-Jacobi sweeps, from -> dst -> the level's other buffer
+// -> dst ..., with the linear part of the fill; returns the buffer that holds
+// the last one (`from` when there are none).  from == nullptr: from zero.
+// The first sweep into a buffer writes every cell of it, later ones those
+// they update and fill.
+float *VCycleMG::smooth_fast_f(int level, const double *b64, const float *b32, int sweeps, float *from, float *dst) {
     Domain &d = m_domain;
-    double ax, ay, az, beta;
-    coeffs(level, &ax, &ay, &az, &beta);
     const LevelDesc &Ld = d.level(level);
     const BCView V = d.bc_view(level, P, true);
-    const int n = mixed_sweep_count(sweeps);
-    const double w = m_mixed_weight > 0.0 ? m_mixed_weight : m_s.smoother.w;
-    auto sweep = [&](bool first, float *dst, const float *src) {
+    const k::MgSweep c = mixed_sweep(level);
+    float *src = from;
+    for (int i = 0; i < sweeps; i++) {
         d.timed("jacobi_mg32", level, [&] {
-            if (b64) k::jacobi_bc<float, double>(d.stream(), Ld, V, first, dst, src, b64, ax, ay, az, beta, kDsign, w);
-            else k::jacobi_bc<float, float>(d.stream(), Ld, V, first, dst, src, b32, ax, ay, az, beta, kDsign, w);
+            const bool first = i < 2;
+            if (b64)
+                k::jacobi_bc<float, double>(d.stream(), Ld, V, first, dst, src, b64, c.ax, c.ay, c.az, c.beta, c.dsign,
+                                            c.w);
+            else
+                k::jacobi_bc<float, float>(d.stream(), Ld, V, first, dst, src, b32, c.ax, c.ay, c.az, c.beta, c.dsign,
+                                           c.w);
         });
-    };
-    // from_zero: tmp is zero and the first sweep does not read it; after
-    // the first sweep tmp is free and the sweeps alternate err1 and tmp.
-    // first_done: the first sweep's result is already in
-    // first_sweep_target(level) (restrict_sweep0)
-    float *src = from_zero ? nullptr : m_tmpf[level];
-    int m = n;
-    if (n % 2 == 0 && n > 0) {
-        if (!first_done) sweep(true, m_scrf[level], src);
-        src = m_scrf[level];
-        m = n - 1;
-        first_done = false;
-    }
-    float *dst = m_err1f[level];
-    for (int i = 0; i < m; i++) {
-        if (!(i == 0 && first_done)) sweep(i == 0, dst, src);
         src = dst;
         dst = dst == m_err1f[level] ? m_tmpf[level] : m_err1f[level];
     }
+    return src;
 }
 
 namespace {
@@ -212,6 +203,51 @@ void VCycleMG::prepare_direct() {
     }
 }
 
+void VCycleMG::upload_direct(const std::vector<double> &inv, const std::vector<uint64_t> &cells) {
+    Domain &d = m_domain;
+    const int f = m_tail_first;
+    const size_t n = cells.size(), size = static_cast<size_t>(d.level(f).size);
+    std::vector<int32_t> map(size);
+    ARTSS_HIP(hipMemcpy(map.data(), d.mg_fill(f).src_of, sizeof(int32_t) * size, hipMemcpyDeviceToHost));
+    std::vector<uint32_t> table(n + n + 1, 0), row_of(size, 0);
+    for (size_t r = 0; r < n; r++) {
+        table[r] = static_cast<uint32_t>(cells[r]);
+        row_of[cells[r]] = static_cast<uint32_t>(r);
+    }
+    auto filled = [&](size_t c, size_t *src) {
+        *src = static_cast<size_t>(map[c] < 0 ? -static_cast<long long>(map[c]) : map[c]) - 1;
+        return map[c] != 0 && *src != c && map[*src] == static_cast<int32_t>(*src + 1);
+    };
+    size_t src = 0;
+    std::vector<uint32_t> count(n + 1, 0);
+    for (size_t c = 0; c < size; c++)
+        if (filled(c, &src)) count[row_of[src] + 1]++;
+    for (size_t r = 0; r < n; r++) count[r + 1] += count[r];
+    std::copy(count.begin(), count.end(), table.begin() + static_cast<std::ptrdiff_t>(n));
+    table.resize(table.size() + count[n]);
+    for (size_t c = 0; c < size; c++)
+        if (filled(c, &src)) {
+            const int32_t to = static_cast<int32_t>(map[c] < 0 ? -static_cast<long long>(c + 1) : c + 1);
+            table[2 * n + 1 + count[row_of[src]]++] = static_cast<uint32_t>(to);
+        }
+    ARTSS_HIP(hipMalloc(&m_direct, sizeof(double) * n * n));
+    ARTSS_HIP(hipMalloc(&m_direct_cells, sizeof(uint32_t) * table.size()));
+    ARTSS_HIP(hipMemcpy(m_direct, inv.data(), sizeof(double) * n * n, hipMemcpyHostToDevice));
+    ARTSS_HIP(hipMemcpy(m_direct_cells, table.data(), sizeof(uint32_t) * table.size(), hipMemcpyHostToDevice));
+    m_direct_n = static_cast<int>(n);
+}
+
+// err1[f] = the exact solve for res1[f], with the linear part of the fill
+// (the restriction before zeroed err1[f])
+void VCycleMG::apply_direct() {
+    const int f = m_tail_first;
+    m_domain.timed("coarse_direct", f, [&] {
+        const uint32_t *ptr = m_direct_cells + m_direct_n;
+        k::dense_apply(m_domain.stream(), m_direct_n, m_direct, m_direct_cells, ptr,
+                       reinterpret_cast<const int32_t *>(ptr + m_direct_n + 1), m_res1[f]->data, m_err1[f]->data);
+    });
+}
+
 // Column j of K is (e_j - J e_j) / beta on the fluid cells, J e_j one
 // Jacobi sweep (weight 1, b = 0) of e_j carrying its linear fill: the sweep
 // gives beta N e_j, N the neighbour sum, and the Jacobi iteration's fixed
@@ -277,13 +313,7 @@ bool VCycleMG::build_direct() {
     std::vector<double> inv;
     if (!invert_dense(K, n, inv)) return false;
     for (double &v : inv) v *= kDsign;
-    std::vector<uint32_t> idx(N);
-    for (size_t i = 0; i < N; i++) idx[i] = static_cast<uint32_t>(cells[i]);
-    ARTSS_HIP(hipMalloc(&m_direct, sizeof(double) * N * N));
-    ARTSS_HIP(hipMalloc(&m_direct_cells, sizeof(uint32_t) * N));
-    ARTSS_HIP(hipMemcpy(m_direct, inv.data(), sizeof(double) * N * N, hipMemcpyHostToDevice));
-    ARTSS_HIP(hipMemcpy(m_direct_cells, idx.data(), sizeof(uint32_t) * N, hipMemcpyHostToDevice));
-    m_direct_n = n;
+    upload_direct(inv, cells);
     return true;
 }
 
@@ -359,13 +389,7 @@ bool VCycleMG::build_galerkin() {
     std::vector<double> inv;
     if (!invert_dense(K, n, inv)) return false;
     for (double &v : inv) v = -v;  // A_c^-1 = -K^-1
-    std::vector<uint32_t> idx(N);
-    for (size_t i = 0; i < N; i++) idx[i] = static_cast<uint32_t>(cells[i]);
-    ARTSS_HIP(hipMalloc(&m_direct, sizeof(double) * N * N));
-    ARTSS_HIP(hipMalloc(&m_direct_cells, sizeof(uint32_t) * N));
-    ARTSS_HIP(hipMemcpy(m_direct, inv.data(), sizeof(double) * N * N, hipMemcpyHostToDevice));
-    ARTSS_HIP(hipMemcpy(m_direct_cells, idx.data(), sizeof(uint32_t) * N, hipMemcpyHostToDevice));
-    m_direct_n = n;
+    upload_direct(inv, cells);
     return true;
 }
 
@@ -397,61 +421,89 @@ void VCycleMG::vcycle_mixed(const double *r) {
     Domain &d = m_domain;
     const int f = m_tail_first;
     hipStream_t s = d.stream();
-    // every level's pre-smoothing starts from zero; below level 0 its first
-    // sweep is fused into the restriction that produces the level's rhs
-    const bool fused_first = mixed_sweep_count(m_mixed_pre) > 0;
+    const int pre = mixed_sweep_count(m_mixed_pre), post = mixed_sweep_count(m_mixed_post);
+    auto other = [&](int level, const float *q) { return q == m_err1f[level] ? m_tmpf[level] : m_err1f[level]; };
+    // the pre-smoothed errors; nullptr: one sweep from zero, which the
+    // kernels that read it evaluate from the right-hand side
+    std::vector<float *> x(static_cast<size_t>(f), nullptr);
     for (int level = 0; level < f; ++level) {
-        const BCView V = d.bc_view(level, P, true);
+        const LevelDesc &Lf = d.level(level), &Lc = d.level(level + 1);
+        const MgFill F = d.mg_fill(level);
         const double *b64 = level == 0 ? r : nullptr;
         const float *b32 = level == 0 ? nullptr : m_res1f[level];
-        smooth_fast_f(level, b64, b32, m_mixed_pre, true, level > 0 && fused_first);
-        d.timed("residuum32", level, [&] {
-            if (b64) k::residuum_faces<float, double>(s, d.level(level), V, m_res0f[level], m_err1f[level], b64);
-            else k::residuum_faces<float, float>(s, d.level(level), V, m_res0f[level], m_err1f[level], b32);
-            // the restriction below reads the ghost layer: fill it
-            if (restrict_reads_ghost(level)) k::fill_bc<float>(s, d.level(level), V, m_res0f[level]);
-        });
+        const k::MgSweep c = mixed_sweep(level);
+        const bool ghosts = restrict_reads_ghost(level);
+        float *&xl = x[static_cast<size_t>(level)];
+        if (pre > 1) {
+            // the first two sweeps in one launch
+            xl = m_err1f[level];
+            d.timed("jacobi_mg32", level, [&] {
+                if (b64) k::smooth_first<float, double>(s, Lf, F, c, xl, nullptr, b64);
+                else k::smooth_first<float, float>(s, Lf, F, c, xl, nullptr, b32);
+            });
+            xl = smooth_fast_f(level, b64, b32, pre - 2, xl, other(level, xl));
+        } else if (ghosts) {
+            xl = smooth_fast_f(level, b64, b32, pre, nullptr, m_err1f[level]);
+        }
+        if (ghosts) {
+            d.timed("residuum32", level, [&] {
+                const BCView V = d.bc_view(level, P, true);
+                if (b64) k::residuum_faces<float, double>(s, Lf, V, m_res0f[level], xl, b64);
+                else k::residuum_faces<float, float>(s, Lf, V, m_res0f[level], xl, b32);
+                // the restriction below reads the ghost layer: fill it
+                k::fill_bc<float>(s, Lf, V, m_res0f[level]);
+            });
+            d.timed("restrict32", level, [&] {
+                if (level + 1 < f)
+                    k::restrict_fill<float, float, float>(s, Lc, Lf, m_res1f[level + 1], m_res0f[level],
+                                                          m_tmpf[level + 1]);
+                else
+                    k::restrict_fill<float, double, double>(s, Lc, Lf, m_res1[level + 1]->data, m_res0f[level],
+                                                            m_err1[level + 1]->data);
+            });
+            continue;
+        }
         d.timed("restrict32", level, [&] {
-            if (level + 1 < f && fused_first) {
-                // the next level's first sweep from zero rides along
-                double cx, cy, cz, cb;
-                coeffs(level + 1, &cx, &cy, &cz, &cb);
-                const double w = m_mixed_weight > 0.0 ? m_mixed_weight : m_s.smoother.w;
-                k::restrict_sweep0(s, d.level(level + 1), d.level(level), d.bc_view(level + 1, P, true),
-                                   m_res1f[level + 1], first_sweep_target(level + 1, m_mixed_pre), m_res0f[level], cx,
-                                   cy, cz, cb, kDsign, w);
-            } else if (level + 1 < f)
-                k::restrict_fill<float, float, float>(s, d.level(level + 1), d.level(level), m_res1f[level + 1],
-                                                      m_res0f[level], m_tmpf[level + 1]);
-            else
-                k::restrict_fill<float, double, double>(s, d.level(level + 1), d.level(level), m_res1[level + 1]->data,
-                                                        m_res0f[level], m_err1[level + 1]->data);
+            float *none = nullptr;
+            if (level + 1 < f) {
+                if (b64) k::residuum_restrict<float, double, float>(s, Lc, Lf, F, c, m_res1f[level + 1], none, xl, b64);
+                else k::residuum_restrict<float, float, float>(s, Lc, Lf, F, c, m_res1f[level + 1], none, xl, b32);
+            } else {
+                double *rhs = m_res1[level + 1]->data, *err = m_err1[level + 1]->data;
+                if (b64) k::residuum_restrict<float, double, double>(s, Lc, Lf, F, c, rhs, err, xl, b64);
+                else k::residuum_restrict<float, float, double>(s, Lc, Lf, F, c, rhs, err, xl, b32);
+            }
         });
     }
     if (m_direct) {
-        // restrict_fill zeroed err1[f]; the solve writes its fluid cells, the fill the rest it sets
-        d.timed("coarse_direct", f, [&] {
-            k::dense_apply(s, m_direct_n, m_direct, m_direct_cells, m_res1[f]->data, m_err1[f]->data);
-            k::fill_bc<double>(s, d.level(f), d.bc_view(f, P, true), m_err1[f]->data);
-        });
+        apply_direct();
     } else {
         d.timed("mg_tail", f, [&] {
             mg_tail(s, m_plan_dev + 1, m_res1[f]->data, m_tail_lds_bytes[1], m_tail_box, precond_coarse_iter(),
                     m_mixed_tail, m_mixed_tail > 0 ? m_mixed_weight : 0.0, true, m_pc_tol);
         });
     }
+    const float *coarse = nullptr;  // the level's result (level f: err1[f], FP64)
     for (int level = f; level > 0; --level) {
         const int fine = level - 1;
-        const BCView V = d.bc_view(fine, P, true);
-        d.timed("prolongate32", fine, [&] {
-            if (level == f)
-                k::prolongate_add_bc<float, double>(s, d.level(level), d.level(fine), V, m_tmpf[fine], m_err1f[fine],
-                                                    m_err1[level]->data);
-            else
-                k::prolongate_add_bc<float, float>(s, d.level(level), d.level(fine), V, m_tmpf[fine], m_err1f[fine],
-                                                   m_err1f[level]);
+        const LevelDesc &Lf = d.level(fine), &Lc = d.level(level);
+        const MgFill F = d.mg_fill(fine), Fc = d.mg_fill(level);
+        const double *b64 = fine == 0 ? r : nullptr;
+        const float *b32 = fine == 0 ? nullptr : m_res1f[fine];
+        const k::MgSweep c = mixed_sweep(fine);
+        const float *xl = x[static_cast<size_t>(fine)];
+        float *dst = other(fine, xl);
+        // (one sweep, which adds the correction first)
+        d.timed("jacobi_mg32", fine, [&] {
+            const double *c64 = m_err1[f]->data;
+            if (level == f && b64) k::smooth_corrected<float, double, double>(s, Lf, F, c, dst, xl, b64, Lc, Fc, c64);
+            else if (level == f) k::smooth_corrected<float, float, double>(s, Lf, F, c, dst, xl, b32, Lc, Fc, c64);
+            else if (b64) k::smooth_corrected<float, double, float>(s, Lf, F, c, dst, xl, b64, Lc, Fc, coarse);
+            else k::smooth_corrected<float, float, float>(s, Lf, F, c, dst, xl, b32, Lc, Fc, coarse);
         });
-        smooth_fast_f(fine, fine == 0 ? r : nullptr, fine == 0 ? nullptr : m_res1f[fine], m_mixed_post, false, false);
+        float *y = smooth_fast_f(fine, b64, b32, post - 1, dst, other(fine, dst));
+        coarse = y;
+        if (fine == 0) m_mixed_out = y;
     }
 }
 
@@ -804,24 +856,35 @@ bool VCycleMG::restrict_reads_ghost(int level) const {
     return false;
 }
 
-// Smoothing of err1[level] whose initial iterate (with the fill applied)
-// is in tmp[level]: sweep 1 tmp -> err1 with the copy folded in, then
-// alternating, the last one into err1.
-void VCycleMG::smooth_fast(int level, const double *b) {
+k::MgSweep VCycleMG::fast_sweep(int level) const {
+    k::MgSweep c{};
+    coeffs(level, &c.ax, &c.ay, &c.az, &c.beta);
+    c.dsign = kDsign;
+    c.w = m_s.smoother.w;
+    return c;
+}
+
+// The sweeps after the first of a smoothing (an even number: the effective
+// count is odd): from -> dst -> other -> dst ..., the last one into `last`
+// when that is given; returns the buffer that holds the last one.  The first
+// sweep into a buffer writes every cell of it.
+double *VCycleMG::smooth_fast(int level, const double *b, int sweeps, double *from, double *dst, double *last) {
     Domain &d = m_domain;
-    double ax, ay, az, beta;
-    coeffs(level, &ax, &ay, &az, &beta);
     const LevelDesc &Ld = d.level(level);
     const BCView V = d.bc_view(level, P);
-    const int n = m_s.n_relax;
-    const int effective = (n % 2 == 0 && n > 0) ? n - 1 : n;
-    double *src = m_tmp[level]->data, *dst = m_err1[level]->data;
-    for (int i = 0; i < effective; i++) {
+    const k::MgSweep c = fast_sweep(level);
+    double *src = from;
+    for (int i = 0; i < sweeps; i++) {
+        const bool to_last = last != nullptr && i == sweeps - 1;
+        double *to = to_last ? last : dst;
         d.timed("jacobi_mg", level, [&] {
-            k::jacobi_bc(d.stream(), Ld, V, i == 0, dst, src, b, ax, ay, az, beta, kDsign, m_s.smoother.w);
+            k::jacobi_bc<double, double>(d.stream(), Ld, V, i < 2 || to_last, to, src, b, c.ax, c.ay, c.az, c.beta,
+                                         c.dsign, c.w);
         });
-        std::swap(src, dst);
+        src = to;
+        dst = dst == m_err1[level]->data ? m_tmp[level]->data : m_err1[level]->data;
     }
+    return src;
 }
 
 // VCycleMG::Smooth on err1[level] with launches folded:
@@ -887,43 +950,60 @@ void VCycleMG::vcycle_fused(Field &out, const Field &b) {
     Domain &d = m_domain;
     const int L = m_s.n_level;
     const int f = m_tail_first;
-    // the buffer the smoothing of `level` starts from
-    auto start = [&](int level) -> Field & { return level < f && fast_level(level) ? *m_tmp[level] : *m_err1[level]; };
-    if (f > 0 && fast_level(0)) {
-        // err1 <- out and the two fills of Smooth fold into tmp <- fill(out)
-        d.timed("copy_bc", 0, [&] { k::copy_bc(d.stream(), d.level(0), d.bc_view(0, P), m_tmp[0]->data, out.data); });
-    } else {
-        m_err1[0]->copy_data(out);
-    }
+    const int n = m_s.n_relax;
+    const int effective = (n % 2 == 0 && n > 0) ? n - 1 : n;
+    if (!(f > 0 && fast_level(0))) m_err1[0]->copy_data(out);
     for (int level = 0; level < f; ++level) {
+        const LevelDesc &Ld = d.level(level);
         const double *rhs = level == 0 ? b.data : m_res1[level]->data;
+        double *err = m_err1[level]->data, *tmp = m_tmp[level]->data;
         // at levels > 0 the smoothing starts from zero, which every fill
         // (all values are zero below level 0) maps to zero: fills elided
-        if (fast_level(level)) smooth_fast(level, rhs);
-        else smooth_fused(level, rhs);
-        if (d.bc_idempotent(level, P) && !restrict_reads_ghost(level)) {
-            d.timed("residuum", level, [&] {
-                k::residuum_faces(d.stream(), d.level(level), d.bc_view(level, P), m_res0[level]->data,
-                                  m_err1[level]->data, rhs);
-            });
+        if (fast_level(level)) {
+            const k::MgSweep c = fast_sweep(level);
+            if (level == 0 && !d.bc_values_zero(0, P)) {
+                // err1 <- out and the two fills of Smooth fold into tmp <- fill(out)
+                d.timed("copy_bc", 0, [&] { k::copy_bc(d.stream(), Ld, d.bc_view(0, P), tmp, out.data); });
+                smooth_fast(level, rhs, effective, tmp, err, nullptr);
+            } else if (level == 0) {
+                d.timed("jacobi_mg", level, [&] {
+                    k::smooth_first<double, double>(d.stream(), Ld, d.mg_fill(0), c, err, out.data, rhs);
+                });
+                smooth_fast(level, rhs, effective - 1, err, tmp, nullptr);
+            } else if (effective == 1) {
+                smooth_fast(level, rhs, 1, nullptr, err, nullptr);
+            } else {
+                // the first two sweeps in one launch
+                d.timed("jacobi_mg", level, [&] {
+                    k::smooth_first<double, double>(d.stream(), Ld, d.mg_fill(level), c, tmp, nullptr, rhs);
+                });
+                smooth_fast(level, rhs, effective - 2, tmp, err, nullptr);
+            }
         } else {
-            d.timed("residuum", level, [&] {
-                k::residuum(d.stream(), d.level(level), m_res0[level]->data, m_err1[level]->data, rhs);
-            });
-            d.apply_boundary(m_res0[level]->data, P, level);
+            smooth_fused(level, rhs);
         }
+        double *next_rhs = m_res1[level + 1]->data;
+        // a fast level evaluates its sweep from zero without reading zeros
+        double *next_err = level + 1 < f && fast_level(level + 1) ? nullptr : m_err1[level + 1]->data;
+        if (d.bc_idempotent(level, P) && !restrict_reads_ghost(level)) {
+            d.timed("restrict", level, [&] {
+                k::residuum_restrict<double, double, double>(d.stream(), d.level(level + 1), Ld, MgFill{}, fast_sweep(level),
+                                                             next_rhs, next_err, m_err1[level]->data,
+                                                             rhs);
+            });
+            continue;
+        }
+        d.timed("residuum", level,
+                [&] { k::residuum(d.stream(), Ld, m_res0[level]->data, m_err1[level]->data, rhs); });
+        d.apply_boundary(m_res0[level]->data, P, level);
         d.timed("restrict", level, [&] {
-            k::restrict_fill(d.stream(), d.level(level + 1), d.level(level), m_res1[level + 1]->data,
-                             m_res0[level]->data, start(level + 1).data);
+            k::restrict_fill(d.stream(), d.level(level + 1), Ld, next_rhs, m_res0[level]->data,
+                             next_err ? next_err : m_tmp[level + 1]->data);
         });
     }
     if (f < L && m_precond_call && m_direct && f > 0) {
-        // as GCR's preconditioner: the exact coarse solve of level f
-        // (restrict_fill above zeroed err1[f])
-        d.timed("coarse_direct", f, [&] {
-            k::dense_apply(d.stream(), m_direct_n, m_direct, m_direct_cells, m_res1[f]->data, m_err1[f]->data);
-            k::fill_bc<double>(d.stream(), d.level(f), d.bc_view(f, P, true), m_err1[f]->data);
-        });
+        // as GCR's preconditioner
+        apply_direct();
     } else if (f < L) {
         d.timed("mg_tail", f, [&] {
             if (m_precond_call)
@@ -933,25 +1013,41 @@ void VCycleMG::vcycle_fused(Field &out, const Field &b) {
                 mg_tail(d.stream(), m_plan_dev, f == 0 ? b.data : m_res1[f]->data, m_tail_lds_bytes[0], m_tail_box);
         });
     }
+    // the result of the level below, err1 where a fast level did not leave it
+    // in its other buffer
+    const double *coarse = m_err1[f]->data;
     for (int level = f; level > 0; --level) {
         const int fine = level - 1;
         const double *rhs = fine == 0 ? b.data : m_res1[fine]->data;
         if (level != L && fast_level(fine)) {
-            d.timed("prolongate", fine, [&] {
-                k::prolongate_add_bc(d.stream(), d.level(level), d.level(fine), d.bc_view(fine, P),
-                                     m_tmp[fine]->data, m_err1[fine]->data, m_err1[level]->data);
+            // the last sweep of level 0 writes `out`
+            double *last = fine == 0 ? out.data : nullptr;
+            if (fine == 0 && !d.bc_values_zero(0, P)) {
+                d.timed("prolongate", fine, [&] {
+                    k::prolongate_add_bc(d.stream(), d.level(level), d.level(fine), d.bc_view(fine, P),
+                                         m_tmp[fine]->data, m_err1[fine]->data, coarse);
+                });
+                coarse = smooth_fast(fine, rhs, effective, m_tmp[fine]->data, m_err1[fine]->data, last);
+                continue;
+            }
+            double *dst = fine == 0 && effective == 1 ? out.data : m_tmp[fine]->data;
+            // (one sweep, which adds the correction first)
+            d.timed("jacobi_mg", fine, [&] {
+                k::smooth_corrected<double, double, double>(d.stream(), d.level(fine), d.mg_fill(fine), fast_sweep(fine),
+                                                            dst, m_err1[fine]->data, rhs, d.level(level),
+                                                            d.mg_fill(level), coarse);
             });
-            smooth_fast(fine, rhs);
+            coarse = smooth_fast(fine, rhs, effective - 1, dst, m_err1[fine]->data, last);
             continue;
         }
         if (d.bc_idempotent(fine, P)) {
             d.timed("prolongate", fine, [&] {
                 k::prolongate_add(d.stream(), d.level(level), d.level(fine), m_err1[fine]->data,
-                                  m_err1[level]->data);
+                                  coarse);
             });
         } else {
             d.timed("prolongate", fine, [&] {
-                k::prolongate(d.stream(), d.level(level), d.level(fine), m_err0[fine]->data, m_err1[level]->data);
+                k::prolongate(d.stream(), d.level(level), d.level(fine), m_err0[fine]->data, coarse);
             });
             d.apply_boundary(m_err0[fine]->data, P, fine);
             *m_err1[fine] += *m_err0[fine];
@@ -962,8 +1058,9 @@ void VCycleMG::vcycle_fused(Field &out, const Field &b) {
         } else {
             smooth_fused(fine, rhs);
         }
+        coarse = m_err1[fine]->data;
     }
-    out.copy_data(*m_err1[0]);
+    if (coarse != out.data) out.copy_data(*m_err1[0]);
     if (!d.bc_idempotent(0, P)) d.apply_boundary(out.data, out.get_type(), 0);
 }
 

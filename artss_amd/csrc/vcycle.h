@@ -5,6 +5,7 @@
 #include <string>
 #include <vector>
 
+#include "mg_fused.h"
 #include "mg_plan.h"
 #include "operators.h"
 
@@ -73,7 +74,7 @@ class VCycleMG : public IPressure {
     static constexpr int kPrecondCoarseSweeps = 5;
     void set_precond_coarse(double coarse_tol, int max_iter);
     void vcycle_mixed(const double *r);
-    float *mixed_result() const { return m_err1f.empty() ? nullptr : m_err1f[0]; }
+    float *mixed_result() const { return m_mixed_out; }
     // The coarse part of the mixed V-cycle (the levels of the single-workgroup
     // kernel) replaced by the exact solve on its first level, x = K^-1 dsign b
     // with K the level's operator and linear fill, applied as a dense matrix
@@ -106,7 +107,7 @@ class VCycleMG : public IPressure {
     void vcycle_plain(Field &out, const Field &b);
     void vcycle_fused(Field &out, const Field &b);
     void smooth_fused(int level, const double *b);
-    void smooth_fast(int level, const double *b);
+    double *smooth_fast(int level, const double *b, int sweeps, double *from, double *dst, double *last);
     bool fast_level(int level) const;
     // Restrict from `level` reads the fine ghost layer (an axis of one cell)
     bool restrict_reads_ghost(int level) const;
@@ -134,7 +135,8 @@ class VCycleMG : public IPressure {
     int m_tail_lds_bytes[2] = {0, 0};
     int m_tail_box = 0;                 // largest inner box the tail relaxes on
     // FP32 level arrays of the mixed V-cycle (levels above the tail)
-    std::vector<float *> m_err1f, m_tmpf, m_scrf, m_res0f, m_res1f;
+    std::vector<float *> m_err1f, m_tmpf, m_res0f, m_res1f;
+    float *m_mixed_out = nullptr;           // level 0 result of the last mixed V-cycle
     int m_mixed_pre = 0, m_mixed_post = 0;  // sweeps of the mixed V-cycle (0: the XML's)
     double m_mixed_weight = 0.0;            // their Jacobi weight (0: the XML's)
     int m_mixed_tail = 0;                   // n_relax of the tail kernel in the mixed V-cycle (0: the XML's)
@@ -146,16 +148,21 @@ class VCycleMG : public IPressure {
     }
     void alloc_mixed();
     void free_mixed();
-    void smooth_fast_f(int level, const double *b64, const float *b32, int sweeps, bool from_zero, bool first_done);
-    int mixed_sweep_count(int sweeps) const;                  // effective sweeps for a count (0: the XML's)
-    float *first_sweep_target(int level, int sweeps) const;   // buffer the first of them writes
+    float *smooth_fast_f(int level, const double *b64, const float *b32, int sweeps, float *from, float *dst);
+    int mixed_sweep_count(int sweeps) const;  // effective sweeps for a count (0: the XML's)
+    k::MgSweep mixed_sweep(int level) const;
+    k::MgSweep fast_sweep(int level) const;
     bool build_galerkin();
     bool build_direct();
     void free_direct();
     bool m_direct_enabled = true;
     bool m_direct_tried = false;
     double *m_direct = nullptr;           // n x n row-major, dsign K^-1
-    uint32_t *m_direct_cells = nullptr;   // the level's fluid cells (row/column order)
+    // the level's fluid cells (row/column order), then per row the start of the cells the fill sets from its
+    // cell (n + 1 entries) and those cells (k::dense_apply)
+    uint32_t *m_direct_cells = nullptr;
+    void upload_direct(const std::vector<double> &inv, const std::vector<uint64_t> &cells);
+    void apply_direct();
     int m_direct_n = 0;
     bool m_use_graphs = true;
     CycleGraph m_graph[2];  // [0]: V-cycle, [1]: V-cycle + residual
