@@ -111,7 +111,7 @@ struct MgFill {
     // leaves alone.  Eight words each: s + 1 of the cell s whose value the
     // item takes (negative: s is not fluid, it keeps the iterate's value),
     // src_of of its neighbours x + 1, x - 1, y + 1, y - 1, z + 1, z - 1, and
-    // the cell written + 1 (negative: with sign -1)
+    // the cell written + 1 (negative: with sign -1; 0: none)
     const int32_t *items;
     int n_items;
     // face ghosts set from an inner fluid cell: target coordinate and sign

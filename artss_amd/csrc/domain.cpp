@@ -5,9 +5,12 @@
 #include <array>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <unordered_map>
 
 #include "kernels.h"
+#include "mg_fused.h"
+#include "stencil.h"
 
 namespace artss {
 
@@ -148,13 +151,8 @@ Domain::~Domain() {
     (void)hipFree(m_gate);
     (void)hipHostFree(m_gate_host);
     (void)hipHostFree(m_sum_host);
-    (void)hipFree(m_faces_dev);
-    (void)hipFree(m_params_dev);
-    (void)hipFree(m_params_hom_dev);
-    (void)hipFree(m_bits_dev);
+    (void)hipFree(m_tables_dev);
     (void)hipFree(m_mg_dev);
-    (void)hipFree(m_deps_dev);
-    (void)hipFree(m_rest_dev);
     (void)hipStreamDestroy(m_stream);
 }
 
@@ -327,8 +325,6 @@ void Domain::build_boundary_tables() {
     std::vector<uint32_t> bits;
     std::vector<DepGhost> deps;
     std::vector<uint32_t> rest;
-    std::vector<int32_t> mg;
-    m_mg_table.assign(m_levels + 1, MgTable());
     m_idem.assign(m_levels + 1, std::vector<char>(NUMBER_OF_FIELD_TYPES, 0));
     m_face_values_zero.assign(m_levels + 1, std::vector<char>(NUMBER_OF_FIELD_TYPES, 1));
     m_view_bits.assign(m_levels + 1, std::vector<long long>(NUMBER_OF_FIELD_TYPES, 0));
@@ -573,99 +569,37 @@ void Domain::build_boundary_tables() {
                     rest.push_back(static_cast<uint32_t>(g));
                 }
                 m_view_nrest[l][f] = static_cast<long long>(rest.size()) - m_view_rest[l][f];
-                if (f == P && m_levels > 0) {
-                    MgTable &M = m_mg_table[l];
-                    M.map = static_cast<long long>(mg.size());
-                    mg.resize(mg.size() + static_cast<size_t>(L.size), 0);
-                    int32_t *map = &mg[static_cast<size_t>(M.map)];
-                    for (int k = 1; k <= L.n[2]; k++)
-                        for (int j = 1; j <= L.n[1]; j++)
-                            for (int i = 1; i <= L.n[0]; i++)
-                                if (!in_obstacle(L, i, j, k)) {
-                                    const long long c = i + Nx * (j + Ny * static_cast<long long>(k));
-                                    map[c] = static_cast<int32_t>(c + 1);
-                                }
-                    std::vector<long long> own;  // cells written by items
-                    const Wave W0 = m_waves[l][f].empty() ? Wave{0, 0} : m_waves[l][f][0];
-                    for (long long e = W0.offset; e < W0.offset + W0.count; e++) {
-                        const FaceEntry &x = entries[static_cast<size_t>(e)];
-                        const long long src = static_cast<long long>(x.idx) + x.ref;
-                        const bool neg = params[static_cast<size_t>(m_param_offset[l][f] + x.param)].sign < 0.0;
-                        map[x.idx] = static_cast<int32_t>(neg ? -(src + 1) : src + 1);
-                        if (written[x.idx] == 2) own.push_back(x.idx);
-                    }
-                    for (size_t t0 = 0; t0 < ghost_src.size(); t0++) {
-                        const long long g = ghost_cell[t0];
-                        const long long i = g % Nx, j = (g / Nx) % Ny, k = g / (Nx * Ny);
-                        double sign = 1.0;
-                        if (i == 0 || i == Nx - 1) sign *= d.sign[i == 0 ? 0 : 1];
-                        if (j == 0 || j == Ny - 1) sign *= d.sign[j == 0 ? 2 : 3];
-                        if (k == 0 || k == Nz - 1) sign *= d.sign[k == 0 ? 4 : 5];
-                        // (the source is a cell the fill does not write or an obstacle face)
-                        const long long src = ghost_src[t0];
-                        const int32_t e = written[static_cast<size_t>(src)] ? map[src] : static_cast<int32_t>(src + 1);
-                        map[g] = sign < 0.0 ? -e : e;
-                    }
-                    for (long long q = m_view_deps[l][f]; q < m_view_deps[l][f] + m_view_ndeps[l][f]; q++)
-                        own.push_back(deps[static_cast<size_t>(q)].idx);
-                    for (long long q = m_view_rest[l][f]; q < m_view_rest[l][f] + m_view_nrest[l][f]; q++)
-                        own.push_back(rest[static_cast<size_t>(q)]);
-                    if (!shell)
-                        for (long long c = 0; c < L.size; c++) {
-                            const long long i = c % Nx, j = (c / Nx) % Ny, k = c / (Nx * Ny);
-                            if ((i == 0 || j == 0 || k == 0 || i == Nx - 1 || j == Ny - 1 || k == Nz - 1) &&
-                                !written[static_cast<size_t>(c)])
-                                own.push_back(c);
-                        }
-                    M.n_items = static_cast<int>(own.size());
-                    std::vector<int32_t> items(8 * own.size(), 0);
-                    const long long off[6] = {1, -1, Nx, -Nx, Nx * Ny, -Nx * Ny};
-                    for (size_t q = 0; q < own.size(); q++) {
-                        const long long c = own[q];
-                        const int32_t e = map[c];
-                        const long long src = e == 0 ? c : (e < 0 ? -e : e) - 1;
-                        const bool fluid = map[src] == static_cast<int32_t>(src + 1);
-                        items[8 * q] = static_cast<int32_t>(fluid ? src + 1 : -(src + 1));
-                        for (int a = 0; a < 6 && fluid; a++) items[8 * q + 1 + a] = map[src + off[a]];
-                        items[8 * q + 7] = static_cast<int32_t>(e < 0 ? -(c + 1) : c + 1);
-                    }
-                    M.items = static_cast<long long>(mg.size());
-                    mg.insert(mg.end(), items.begin(), items.end());
-                }
             }
         }
     }
     m_face_entries = static_cast<long long>(entries.size());
     if (m_device < 0) return;
-    if (!entries.empty()) {
-        ARTSS_HIP(hipMalloc(&m_faces_dev, sizeof(FaceEntry) * entries.size()));
-        ARTSS_HIP(hipMemcpy(m_faces_dev, entries.data(), sizeof(FaceEntry) * entries.size(), hipMemcpyHostToDevice));
-    }
-    if (!params.empty()) {
-        ARTSS_HIP(hipMalloc(&m_params_dev, sizeof(FaceParam) * params.size()));
-        ARTSS_HIP(hipMemcpy(m_params_dev, params.data(), sizeof(FaceParam) * params.size(), hipMemcpyHostToDevice));
-        // the same table with every boundary value zero (linear part of the fill)
-        std::vector<FaceParam> hom = params;
-        for (FaceParam &q : hom) q.value = 0.0;
-        ARTSS_HIP(hipMalloc(&m_params_hom_dev, sizeof(FaceParam) * hom.size()));
-        ARTSS_HIP(hipMemcpy(m_params_hom_dev, hom.data(), sizeof(FaceParam) * hom.size(), hipMemcpyHostToDevice));
-    }
-    if (!bits.empty()) {
-        ARTSS_HIP(hipMalloc(&m_bits_dev, sizeof(uint32_t) * bits.size()));
-        ARTSS_HIP(hipMemcpy(m_bits_dev, bits.data(), sizeof(uint32_t) * bits.size(), hipMemcpyHostToDevice));
-    }
-    if (!mg.empty()) {
-        ARTSS_HIP(hipMalloc(&m_mg_dev, sizeof(int32_t) * mg.size()));
-        ARTSS_HIP(hipMemcpy(m_mg_dev, mg.data(), sizeof(int32_t) * mg.size(), hipMemcpyHostToDevice));
-    }
-    if (!deps.empty()) {
-        ARTSS_HIP(hipMalloc(&m_deps_dev, sizeof(DepGhost) * deps.size()));
-        ARTSS_HIP(hipMemcpy(m_deps_dev, deps.data(), sizeof(DepGhost) * deps.size(), hipMemcpyHostToDevice));
-    }
-    if (!rest.empty()) {
-        ARTSS_HIP(hipMalloc(&m_rest_dev, sizeof(uint32_t) * rest.size()));
-        ARTSS_HIP(hipMemcpy(m_rest_dev, rest.data(), sizeof(uint32_t) * rest.size(), hipMemcpyHostToDevice));
-    }
+    // one allocation: the fills read several of these tables in a chain, and
+    // each allocation is a page of its own to translate on a first call
+    std::vector<FaceParam> hom = params;  // every boundary value zero (linear part of the fill)
+    for (FaceParam &q : hom) q.value = 0.0;
+    size_t bytes = 0;
+    auto place = [&](size_t n) {
+        const size_t o = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return o;
+    };
+    const size_t o_faces = place(sizeof(FaceEntry) * entries.size()), o_params = place(sizeof(FaceParam) * params.size()),
+                 o_hom = place(sizeof(FaceParam) * hom.size()), o_bits = place(sizeof(uint32_t) * bits.size()),
+                 o_deps = place(sizeof(DepGhost) * deps.size()), o_rest = place(sizeof(uint32_t) * rest.size());
+    if (bytes == 0) return;
+    ARTSS_HIP(hipMalloc(&m_tables_dev, bytes));
+    auto upload = [&](auto *&dev, const auto &host, size_t o) {
+        if (host.empty()) return;
+        dev = reinterpret_cast<std::remove_reference_t<decltype(dev)>>(m_tables_dev + o);
+        ARTSS_HIP(hipMemcpy(dev, host.data(), sizeof(host[0]) * host.size(), hipMemcpyHostToDevice));
+    };
+    upload(m_faces_dev, entries, o_faces);
+    upload(m_params_dev, params, o_params);
+    upload(m_params_hom_dev, hom, o_hom);
+    upload(m_bits_dev, bits, o_bits);
+    upload(m_deps_dev, deps, o_deps);
+    upload(m_rest_dev, rest, o_rest);
 }
 
 BCView Domain::bc_view(int level, int ft, bool homogeneous) const {
@@ -689,9 +623,34 @@ BCView Domain::bc_view(int level, int ft, bool homogeneous) const {
     return v;
 }
 
+void Domain::build_mg_fills() {
+    if (m_mg_dev != nullptr || m_device < 0) return;
+    m_mg_table.assign(static_cast<size_t>(m_levels) + 1, MgTable());
+    long long words = 0;
+    for (int l = 0; l <= m_levels; l++) {
+        const long long size = m_level[l].size;
+        if (!m_idem[l][P] || size >= (1LL << 31) - 1) continue;
+        MgTable &M = m_mg_table[l];
+        const BCView V = bc_view(l, P, true);
+        M.n_items = static_cast<int>(dev::bc_items_grid(V) + (V.shell_filled ? 0 : ghost_cells(l)));
+        M.map = words;
+        M.items = words + (size + 7) / 8 * 8;
+        words = M.items + 8LL * M.n_items;
+    }
+    if (words == 0) return;
+    ARTSS_HIP(hipMalloc(&m_mg_dev, sizeof(int32_t) * static_cast<size_t>(words)));
+    for (int l = 0; l <= m_levels; l++) {
+        const MgTable &M = m_mg_table[static_cast<size_t>(l)];
+        if (M.map >= 0)
+            k::build_mg_fill(m_stream, m_level[l], bc_view(l, P, true), m_mg_dev + M.map, m_mg_dev + M.items, M.n_items);
+    }
+    ARTSS_HIP(hipStreamSynchronize(m_stream));
+}
+
 MgFill Domain::mg_fill(int level) const {
+    if (m_mg_dev == nullptr || m_mg_table[static_cast<size_t>(level)].map < 0)
+        throw std::logic_error("mg_fill of a level without an idempotent fill");
     const MgTable &M = m_mg_table[static_cast<size_t>(level)];
-    if (M.map < 0 || m_mg_dev == nullptr) throw std::logic_error("mg_fill of a level without an idempotent fill");
     MgFill f{};
     f.src_of = m_mg_dev + M.map;
     f.items = m_mg_dev + M.items;
@@ -721,11 +680,36 @@ long long Domain::ghost_cells(int level) const {
 void Domain::apply_boundary(double *f, int ft, int level, const int *gate) {
     require_device();
     if (ft < 0 || ft >= NUMBER_OF_FIELD_TYPES) return;  // UNKNOWN_FIELD has no boundary data
+    // an idempotent fill is one launch (its ghosts that read an obstacle face
+    // evaluate that face): 6 instead of 10 us at 256x128x128, either
+    // little more than a launch
+    if (gate == nullptr && m_idem[level][ft]) {
+        apply_boundaries(&f, &ft, 1, level);
+        return;
+    }
     for (const Wave &w : m_waves[level][ft])
         timed("bc_faces", level, [&] {
             k::bc_faces(m_stream, m_faces_dev + w.offset, w.count, m_params_dev + m_param_offset[level][ft], f, gate);
         });
     timed("bc_domain", level, [&] { k::bc_domain(m_stream, m_level[level], m_dom_bc[level][ft], f, gate); });
+}
+
+void Domain::apply_boundaries(double *const *f, const int *field_types, int count, int level) {
+    require_device();
+    BCView V[k::kMaxFills];
+    double *fields[k::kMaxFills];
+    int n = 0;
+    for (int q = 0; q < count; q++) {
+        const int ft = field_types[q];
+        if (ft < 0 || ft >= NUMBER_OF_FIELD_TYPES) continue;  // UNKNOWN_FIELD has no boundary data
+        if (!m_idem[level][ft]) {
+            apply_boundary(f[q], ft, level);
+            continue;
+        }
+        V[n] = bc_view(level, ft);
+        fields[n++] = f[q];
+    }
+    if (n > 0) timed("bc_merged", level, [&] { k::fill_bcs(m_stream, m_level[level], V, fields, n); });
 }
 
 void Domain::apply_boundary_merged(double *f, int ft, int level) {

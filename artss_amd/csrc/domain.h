@@ -81,6 +81,8 @@ class Domain {
     // faces first, then the six domain patches.
     // gate (optional): the fill's kernels do nothing while *gate != 0 (k::IterGate)
     void apply_boundary(double *f, int field_type, int level, const int *gate = nullptr);
+    // ... on `count` different fields (up to k::kMaxFills)
+    void apply_boundaries(double *const *f, const int *field_types, int count, int level);
 
     // A fill is simple when no write of it reads a cell that any of its
     // writes changes: it then needs one wave of face writes, faces and
@@ -96,6 +98,7 @@ class Domain {
     // the pressure-type fill of a multigrid level whose fill is idempotent,
     // with every value taken as zero
     MgFill mg_fill(int level) const;
+    void build_mg_fills();  // its tables, once, before the first mg_fill (not during stream capture)
     BCView bc_view(int level, int field_type, bool homogeneous = false) const;
     // the fill has no non-zero boundary value (it is linear)
     bool bc_values_zero(int level, int field_type) const;
@@ -199,6 +202,7 @@ class Domain {
     FaceParam *m_params_hom_dev = nullptr;
     std::vector<std::vector<long long>> m_view_bits, m_view_deps, m_view_ndeps, m_view_rest, m_view_nrest;
     uint32_t *m_rest_dev = nullptr;
+    char *m_tables_dev = nullptr;  // the allocation the tables of the fills lie in
     uint32_t *m_bits_dev = nullptr;
     int32_t *m_mg_dev = nullptr;  // MgFill tables of the pressure-type fills, per level the map, then the items
     struct MgTable {

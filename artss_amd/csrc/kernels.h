@@ -48,8 +48,9 @@ void bc_merged(hipStream_t s, const LevelDesc &L, const DomainBC &bc, const Face
                const FaceParam *p, double *f);
 
 // ---- SLAdvect::advect (SLAdvect.cpp:71-163) ----
+// V (an idempotent fill; out none of the arrays read): with the fill after it
 void sl_advect(hipStream_t s, const LevelDesc &L, double dt, double *out, const double *in, const double *u,
-               const double *v, const double *w);
+               const double *v, const double *w, const BCView *V = nullptr);
 
 // ---- Jacobi diffusion (JacobiDiffuse.cpp) with fused update-size partials ----
 // plain level-0 form divides by rb (:241-249), turbulent form (:345-362) when ev != nullptr.
@@ -136,6 +137,9 @@ void prolongate_add_bc(hipStream_t s, const LevelDesc &Lc, const LevelDesc &Lf, 
                        const Tf *fine, const Tc *coarse);
 template <typename T>
 void fill_bc(hipStream_t s, const LevelDesc &L, const BCView &V, T *f);
+// the idempotent fills of up to kMaxFills different fields of a level in one launch
+constexpr int kMaxFills = 3;
+void fill_bcs(hipStream_t s, const LevelDesc &L, const BCView *V, double *const *f, int count);
 
 // ---- reductions ----
 int partial_count(const LevelDesc &L);  // number of partial slots a level-wide kernel writes

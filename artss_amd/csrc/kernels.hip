@@ -210,58 +210,70 @@ __global__ void k_bc_merged(LevelDesc L, DomainBC bc, const FaceEntry *__restric
 // ------------------------------------------------------------------ advection
 // SLAdvect.cpp:71-163.  fmod(C, 1) of a finite C > 0 equals C - trunc(C)
 // exactly (the difference is representable, Sterbenz), so no library call.
-__global__ void k_sl_advect(LevelDesc L, double dtx, double dty, double dtz, double *__restrict__ out,
-                            const double *__restrict__ in, const double *__restrict__ u,
-                            const double *__restrict__ v, const double *__restrict__ w) {
-    int ci, cj, ck;
-    if (!inner_cell(L, ci, cj, ck)) return;
-    const long long idx = lin(L, ci, cj, ck);
+struct AdvectArgs {
+    double dtx, dty, dtz;
+    const double *in, *u, *v, *w;
+};
+__device__ __forceinline__ double sl_value(const LevelDesc &L, const AdvectArgs &a, int ci, int cj, int ck,
+                                           long long idx) {
+    const double *__restrict__ in = a.in;
     const double eps = 1e-6;
-    const long i = ci, j = cj, k = ck;
-    const double Ci = dtx * u[idx], Cj = dty * v[idx], Ck = dtz * w[idx];
-    long i0 = i, i1 = i, j0 = j, j1 = j, k0 = k, k1 = k;
+    const int i = ci, j = cj, k = ck;
+    const double Ci = a.dtx * a.u[idx], Cj = a.dty * a.v[idx], Ck = a.dtz * a.w[idx];
+    int i0 = i, i1 = i, j0 = j, j1 = j, k0 = k, k1 = k;
     double r = 1, s = 1, t = 1;
-    // cell shift (long)C; |C| is capped at 1e12 only so the cast cannot
-    // overflow (the clamp to the inner range below already covers any such C)
-    auto shift = [](double C) { return static_cast<long>(fmin(fmax(C, -1e12), 1e12)); };
+    // cell shift (long)C; |C| is capped at 1e9 only so that neither the cast
+    // nor the difference can overflow (the clamp to the inner range below
+    // already covers any such C)
+    auto shift = [](double C) { return static_cast<int>(fmin(fmax(C, -1e9), 1e9)); };
     if (Ci > eps) {
-        i0 = max(1L, i - shift(Ci));
+        i0 = max(1, i - shift(Ci));
         i1 = i0 - 1;
         r = Ci - trunc(Ci);
     } else if (Ci < -eps) {
-        i0 = min(static_cast<long>(L.n[0]), i - shift(Ci));
+        i0 = min(L.n[0], i - shift(Ci));
         i1 = i0 + 1;
         r = (-Ci) - trunc(-Ci);
     }
     if (Cj > eps) {
-        j0 = max(1L, j - shift(Cj));
+        j0 = max(1, j - shift(Cj));
         j1 = j0 - 1;
         s = Cj - trunc(Cj);
     } else if (Cj < -eps) {
-        j0 = min(static_cast<long>(L.n[1]), j - shift(Cj));
+        j0 = min(L.n[1], j - shift(Cj));
         j1 = j0 + 1;
         s = (-Cj) - trunc(-Cj);
     }
     if (Ck > eps) {
-        k0 = max(1L, k - shift(Ck));
+        k0 = max(1, k - shift(Ck));
         k1 = k0 - 1;
         t = Ck - trunc(Ck);
     } else if (Ck < -eps) {
-        k0 = min(static_cast<long>(L.n[2]), k - shift(Ck));
+        k0 = min(L.n[2], k - shift(Ck));
         k1 = k0 + 1;
         t = (-Ck) - trunc(-Ck);
     }
-    const double d000 = in[lin(L, i0, j0, k0)], d100 = in[lin(L, i1, j0, k0)];
-    const double d010 = in[lin(L, i0, j1, k0)], d110 = in[lin(L, i1, j1, k0)];
-    const double d001 = in[lin(L, i0, j0, k1)], d101 = in[lin(L, i1, j0, k1)];
-    const double d011 = in[lin(L, i0, j1, k1)], d111 = in[lin(L, i1, j1, k1)];
+    const unsigned nj = static_cast<unsigned>(L.N[0]), nk = nj * static_cast<unsigned>(L.N[1]);
+    const unsigned x0 = static_cast<unsigned>(i0), x1 = static_cast<unsigned>(i1), y0 = nj * static_cast<unsigned>(j0),
+                   y1 = nj * static_cast<unsigned>(j1), z0 = nk * static_cast<unsigned>(k0),
+                   z1 = nk * static_cast<unsigned>(k1);
+    const double d000 = in[x0 + y0 + z0], d100 = in[x1 + y0 + z0];
+    const double d010 = in[x0 + y1 + z0], d110 = in[x1 + y1 + z0];
+    const double d001 = in[x0 + y0 + z1], d101 = in[x1 + y0 + z1];
+    const double d011 = in[x0 + y1 + z1], d111 = in[x1 + y1 + z1];
     const double r100 = d000 + r * (d100 - d000);
     const double r110 = d010 + r * (d110 - d010);
     const double r101 = d001 + r * (d101 - d001);
     const double r111 = d011 + r * (d111 - d011);
     const double s110 = r100 + s * (r110 - r100);
     const double s111 = r101 + s * (r111 - r101);
-    out[idx] = s110 + t * (s111 - s110);
+    return s110 + t * (s111 - s110);
+}
+__global__ void k_sl_advect(LevelDesc L, AdvectArgs a, double *__restrict__ out) {
+    int i, j, k;
+    if (!inner_cell(L, i, j, k)) return;
+    const long long idx = lin(L, i, j, k);
+    out[idx] = sl_value(L, a, i, j, k, idx);
 }
 
 // ------------------------------------------------------------------ Jacobi
@@ -1208,7 +1220,47 @@ __global__ void k_dense_apply(int n, const double *__restrict__ M, const uint32_
     }
 }
 
+// The advected field with its fill (idempotent fills, out none of the
+// arrays read): the two launches of the fill took nearly as long as the
+// advection on boxes of a million cells (13 + 9 us at 150x70x93, now 13; the
+// whole call 28.6, now 22.3), and at 16^3 the call is all launches (17.8, now
+// 14.9).  The advection itself is bound by memory (256x128x128: 39 us for
+// five arrays).
+// The items' workgroups come first: an item is a chain of four loads, which
+// as the last to start were 4 us of the launch.
+__global__ void k_sl_advect_bc(LevelDesc L, BCView V, int items_z, AdvectArgs a, double *__restrict__ out) {
+    if (static_cast<int>(blockIdx.z) < items_z) {
+        auto val = [&](long long c) {
+            int ci, cj, ck;
+            return is_inner(L, c, ci, cj, ck) ? sl_value(L, a, ci, cj, ck, c) : out[c];
+        };
+        dev::bc_item<double, decltype(val), true>(L, V, item_index(0), out, val);
+        return;
+    }
+    // contiguous runs of workgroups per XCD (main_block)
+    const unsigned gx = gridDim.x, gy = gridDim.y, main = gx * gy * (gridDim.z - static_cast<unsigned>(items_z));
+    const unsigned id = blockIdx.x + gx * (blockIdx.y + gy * (blockIdx.z - static_cast<unsigned>(items_z))), per = main / 8u;
+    const unsigned nid = id < per * 8u ? (id % 8u) * per + id / 8u : id;
+    const int i = 1 + static_cast<int>(nid % gx) * BX + static_cast<int>(threadIdx.x),
+              j = 1 + static_cast<int>(nid / gx % gy) * BY + static_cast<int>(threadIdx.y),
+              k = 1 + static_cast<int>(nid / (gx * gy));
+    if (i > L.n[0] || j > L.n[1] || in_obstacle(L, i, j, k)) return;
+    const long long idx = lin(L, i, j, k);
+    const double v = sl_value(L, a, i, j, k, idx);
+    out[idx] = v;
+    dev::face_ghosts(L, V, out, idx, i, j, k, v);
+}
+
 // One idempotent fill in a single launch (faces, ghosts, dependent ghosts)
+// (several fields of a level at once: one row of workgroups each)
+struct FillJobs {
+    BCView V[kMaxFills];
+    double *f[kMaxFills];
+};
+__global__ void k_fill_bcs(LevelDesc L, FillJobs jobs) {
+    double *f = jobs.f[blockIdx.y];
+    dev::bc_item(L, jobs.V[blockIdx.y], blockIdx.x * 256LL + threadIdx.x, f, [&](long long c) { return f[c]; });
+}
 template <typename T>
 __global__ void k_fill_bc(LevelDesc L, BCView V, T *__restrict__ f) {
     dev::bc_item(L, V, blockIdx.x * 256LL + threadIdx.x, f, [&](long long c) { return f[c]; });
@@ -1330,10 +1382,13 @@ __global__ void k_projection(LevelDesc L, double hx, double hy, double hz, doubl
 __global__ void k_smagorinsky(LevelDesc L, double rdx, double rdy, double rdz, double cdd, double *__restrict__ ev,
                               const double *__restrict__ u, const double *__restrict__ v,
                               const double *__restrict__ w) {
-    int i, j, k;
-    if (!inner_cell(L, i, j, k)) return;
-    const long long idx = lin(L, i, j, k);
-    const long long ni = 1, nj = L.N[0], nk = static_cast<long long>(L.N[0]) * L.N[1];
+    int bx, by, bz;
+    main_block(static_cast<int>(gridDim.z), bx, by, bz);
+    const int i = 1 + bx * BX + static_cast<int>(threadIdx.x), j = 1 + by * BY + static_cast<int>(threadIdx.y),
+              k = 1 + bz;
+    if (i > L.n[0] || j > L.n[1]) return;
+    const unsigned nj = static_cast<unsigned>(L.N[0]), nk = nj * static_cast<unsigned>(L.N[1]), ni = 1;
+    const unsigned idx = static_cast<unsigned>(i) + nj * static_cast<unsigned>(j) + nk * static_cast<unsigned>(k);
     const double S11 = (u[idx + ni] - u[idx - ni]) * 0.5 * rdx;
     const double S22 = (v[idx + nj] - v[idx - nj]) * 0.5 * rdy;
     const double S33 = (w[idx + nk] - w[idx - nk]) * 0.5 * rdz;
@@ -1342,7 +1397,8 @@ __global__ void k_smagorinsky(LevelDesc L, double rdx, double rdy, double rdz, d
     const double S23 = 0.5 * ((v[idx + nk] - v[idx - nk]) * 0.5 * rdz + (w[idx + nj] - w[idx - nj]) * 0.5 * rdy);
     const double S_bar = sqrt(2. * (S11 * S11 + S22 * S22 + S33 * S33 + 2. * (S12 * S12) + 2. * (S13 * S13) +
                                     2. * (S23 * S23)));
-    ev[idx] = cdd * S_bar;
+    // (tested last: the loads are on their way meanwhile)
+    if (!in_obstacle(L, i, j, k)) ev[idx] = cdd * S_bar;
 }
 
 // ------------------------------------------------------------------ sources
@@ -1424,8 +1480,15 @@ void bc_merged(hipStream_t s, const LevelDesc &L, const DomainBC &bc, const Face
 }
 
 void sl_advect(hipStream_t s, const LevelDesc &L, double dt, double *out, const double *in, const double *u,
-               const double *v, const double *w) {
-    k_sl_advect<<<inner_grid(L), block(), 0, s>>>(L, dt / L.h[0], dt / L.h[1], dt / L.h[2], out, in, u, v, w);
+               const double *v, const double *w, const BCView *V) {
+    const AdvectArgs a{dt / L.h[0], dt / L.h[1], dt / L.h[2], in, u, v, w};
+    if (V == nullptr) {
+        k_sl_advect<<<inner_grid(L), block(), 0, s>>>(L, a, out);
+        return;
+    }
+    const dim3 g = inner_grid(L);
+    const dim3 gi = with_items(g, dev::bc_items_grid(*V));
+    k_sl_advect_bc<<<gi, block(), 0, s>>>(L, *V, static_cast<int>(gi.z - g.z), a, out);
 }
 
 void jacobi_diffuse_step(hipStream_t s, const LevelDesc &L, double *out, const double *in, const double *b,
@@ -1640,6 +1703,18 @@ void prolongate_add_bc(hipStream_t s, const LevelDesc &Lc, const LevelDesc &Lf, 
 template void prolongate_add_bc<double, double>(hipStream_t, const LevelDesc &, const LevelDesc &, const BCView &,
                                                 double *, const double *, const double *);
 
+void fill_bcs(hipStream_t s, const LevelDesc &L, const BCView *V, double *const *f, int count) {
+    if (count < 1 || count > kMaxFills) throw std::invalid_argument("fill_bcs: 1 to kMaxFills fields");
+    FillJobs jobs{};
+    long long n = 0;
+    for (int q = 0; q < count; q++) {
+        jobs.V[q] = V[q];
+        jobs.f[q] = f[q];
+        n = std::max(n, dev::bc_items(V[q]));
+    }
+    if (n == 0) return;
+    k_fill_bcs<<<dim3(static_cast<unsigned>((n + 255) / 256), static_cast<unsigned>(count)), 256, 0, s>>>(L, jobs);
+}
 template <typename T>
 void fill_bc(hipStream_t s, const LevelDesc &L, const BCView &V, T *f) {
     const long long n = dev::bc_items(V);

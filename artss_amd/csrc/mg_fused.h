@@ -9,6 +9,10 @@
 namespace artss {
 namespace k {
 
+// the map and the items (MgFill) of a fill; n_items: its fill items in the
+// form of dev::bc_items_grid, then the ghost cells if the fill leaves some
+void build_mg_fill(hipStream_t s, const LevelDesc &L, const BCView &V, int32_t *map, int32_t *items, int n_items);
+
 // one weighted-Jacobi sweep of a level
 struct MgSweep {
     double ax, ay, az, beta, dsign, w;

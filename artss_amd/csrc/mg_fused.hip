@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(kThreads)
         const T xp = __shfl(v, lane0 + 1, 64), xm = __shfl(v, lane0 + 2, 64), yp = __shfl(v, lane0 + 3, 64),
                 ym = __shfl(v, lane0 + 4, 64), zp = __shfl(v, lane0 + 5, 64), zm = __shfl(v, lane0 + 6, 64);
         const int to = __shfl(e, lane0 + 7, 64);
-        if (l != 0) return;
+        if (l != 0 || to == 0) return;
         if (e > 0) {
             const T out_h = c.beta * (c.dsign * rhs + c.ax * (xp + xm) + c.ay * (yp + ym) + c.az * (zp + zm));
             v = (1 - c.w) * v + c.w * out_h;
@@ -493,6 +493,75 @@ __global__ void __launch_bounds__(kThreads)
     out[cidx] = static_cast<Tout>(static_cast<T>(0.125) * sum);
 }
 
+// ---- MgFill tables, three launches: each reads what the one before wrote
+__global__ void k_map_cells(LevelDesc L, int32_t *__restrict__ map) {
+    const long long n = blockIdx.x * 256LL + threadIdx.x;
+    if (n >= L.size) return;
+    const unsigned u = static_cast<unsigned>(n), Nx = static_cast<unsigned>(L.N[0]), Ny = static_cast<unsigned>(L.N[1]);
+    const int i = static_cast<int>(u % Nx), j = static_cast<int>((u / Nx) % Ny), k = static_cast<int>(u / (Nx * Ny));
+    const bool fluid = i >= 1 && j >= 1 && k >= 1 && i <= L.n[0] && j <= L.n[1] && k <= L.n[2] && !in_obstacle(L, i, j, k);
+    map[n] = fluid ? static_cast<int32_t>(n + 1) : 0;
+}
+__global__ void k_map_faces(BCView V, int32_t *__restrict__ map) {
+    const long long t = blockIdx.x * 256LL + threadIdx.x;
+    if (t >= V.n_faces) return;
+    const FaceEntry e = V.faces[t];
+    const FaceParam q = V.params[e.param];
+    if (!q.active) return;
+    const int32_t src = static_cast<int32_t>(e.idx) + e.ref + 1;
+    map[e.idx] = q.sign < 0.0 ? -src : src;
+}
+__device__ __forceinline__ double ghost_sign(const LevelDesc &L, const DomainBC &bc, long long i, long long j,
+                                             long long k) {
+    return dev::ghost_chain<double>(L, bc, i, j, k, 1.0);  // the values are zero
+}
+__global__ void k_map_ghosts(LevelDesc L, BCView V, int32_t *__restrict__ map) {
+    const long long t = blockIdx.x * 256LL + threadIdx.x;
+    long long i, j, k;
+    if (t >= V.n_ghosts || !dev::ghost_coords(L, t, i, j, k)) return;
+    // (the source is a cell the fill does not write or an obstacle face)
+    const long long src = dev::ghost_source(L, V.bc, i, j, k);
+    const int32_t e = dev::written(V, src) ? map[src] : static_cast<int32_t>(src + 1);
+    map[dev::lin(L, i, j, k)] = ghost_sign(L, V.bc, i, j, k) < 0.0 ? -e : e;
+}
+__global__ void k_map_items(LevelDesc L, BCView V, const int32_t *__restrict__ map, int32_t *__restrict__ items,
+                            int n_items) {
+    const long long q = blockIdx.x * 256LL + threadIdx.x;
+    if (q >= n_items) return;
+    long long t = q, cell = -1;
+    if (t < V.n_faces) {
+        const FaceEntry e = V.faces[t];
+        long long i = e.idx % L.N[0], j = (e.idx / L.N[0]) % L.N[1], k = e.idx / (static_cast<long long>(L.N[0]) * L.N[1]);
+        const bool shell = i == 0 || j == 0 || k == 0 || i == L.N[0] - 1 || j == L.N[1] - 1 || k == L.N[2] - 1;
+        // (a face on the ghost layer is overwritten by the ghosts)
+        if (!(shell && V.n_ghosts != 0)) cell = e.idx;
+    } else if ((t -= V.n_faces) < V.n_rest) {
+        cell = V.rest[t];
+    } else if ((t -= V.n_rest) < V.n_deps) {
+        cell = V.deps[t].idx;
+    } else {
+        long long i, j, k;
+        if (dev::ghost_coords(L, t - V.n_deps, i, j, k) && !dev::written(V, dev::lin(L, i, j, k))) cell = dev::lin(L, i, j, k);
+    }
+    int32_t *out = items + 8 * q;
+    for (int a = 0; a < 8; a++) out[a] = 0;
+    if (cell < 0) return;
+    const int32_t e = map[cell];
+    const long long src = e == 0 ? cell : (e < 0 ? -static_cast<long long>(e) : e) - 1;
+    const bool fluid = map[src] == static_cast<int32_t>(src + 1);
+    const long long nj = L.N[0], nk = nj * L.N[1];
+    out[0] = static_cast<int32_t>(fluid ? src + 1 : -(src + 1));
+    if (fluid) {
+        out[1] = map[src + 1];
+        out[2] = map[src - 1];
+        out[3] = map[src + nj];
+        out[4] = map[src - nj];
+        out[5] = map[src + nk];
+        out[6] = map[src - nk];
+    }
+    out[7] = static_cast<int32_t>(e < 0 ? -(cell + 1) : cell + 1);
+}
+
 template <typename T, typename TB, typename Tc, bool FROM_B, bool COARSE, int TY, int TZ>
 void launch_start(hipStream_t s, const Start<T, TB, Tc> &S, const Boxes &boxes, const MgFill &F, const MgSweep &c,
                   T *dst) {
@@ -519,6 +588,13 @@ void pick_start(hipStream_t s, const Start<T, TB, Tc> &S, const Boxes &boxes, co
 
 }  // namespace
 
+void build_mg_fill(hipStream_t s, const LevelDesc &L, const BCView &V, int32_t *map, int32_t *items, int n_items) {
+    auto blocks = [](long long n) { return static_cast<unsigned>((n + 255) / 256); };
+    k_map_cells<<<blocks(L.size), 256, 0, s>>>(L, map);
+    if (V.n_faces > 0) k_map_faces<<<blocks(V.n_faces), 256, 0, s>>>(V, map);
+    if (V.n_ghosts > 0) k_map_ghosts<<<blocks(V.n_ghosts), 256, 0, s>>>(L, V, map);
+    if (n_items > 0) k_map_items<<<blocks(n_items), 256, 0, s>>>(L, V, map, items, n_items);
+}
 template <typename T, typename TB>
 void smooth_first(hipStream_t s, const LevelDesc &L, const MgFill &F, const MgSweep &c, T *dst, const T *x,
                   const TB *b) {

@@ -23,9 +23,9 @@ void IPressure::projection(Field &out_u, Field &out_v, Field &out_w, const Field
                            const Field &in_w, const Field &in_p, bool sync) {
     k::projection(m_domain.stream(), m_domain.level(0), out_u.data, out_v.data, out_w.data, in_u.data, in_v.data,
                   in_w.data, in_p.data);
-    m_domain.apply_boundary(out_u.data, out_u.get_type(), 0);
-    m_domain.apply_boundary(out_v.data, out_v.get_type(), 0);
-    m_domain.apply_boundary(out_w.data, out_w.get_type(), 0);
+    double *out[3] = {out_u.data, out_v.data, out_w.data};
+    const int types[3] = {out_u.get_type(), out_v.get_type(), out_w.get_type()};
+    m_domain.apply_boundaries(out, types, 3, 0);
     maybe_sync(m_domain, sync);
 }
 
@@ -45,11 +45,17 @@ void ISource::dissipate(Field &out, const Field &in_u, const Field &in_v, const 
 }
 
 void SLAdvect::advect(Field &out, const Field &in, const Field &u, const Field &v, const Field &w, bool sync) {
+    const int ft = out.get_type();
+    // the fill's items read the operands again after other cells of `out` are
+    // written: it rides along only where `out` is none of them
+    const bool apart = out.data != in.data && out.data != u.data && out.data != v.data && out.data != w.data;
+    const bool fused = apart && ft >= 0 && ft < NUMBER_OF_FIELD_TYPES && m_domain.bc_idempotent(0, ft);
+    const BCView V = fused ? m_domain.bc_view(0, ft) : BCView{};
     m_domain.timed("sl_advect", 0, [&] {
         k::sl_advect(m_domain.stream(), m_domain.level(0), m_domain.settings().dt, out.data, in.data, u.data,
-                     v.data, w.data);
+                     v.data, w.data, fused ? &V : nullptr);
     });
-    m_domain.apply_boundary(out.data, out.get_type(), 0);
+    if (!fused) m_domain.apply_boundary(out.data, ft, 0);
     maybe_sync(m_domain, sync);
 }
 
@@ -307,13 +313,17 @@ void ExplicitEulerSource::add_source(Field &out_x, Field &out_y, Field &out_z, c
     const double dt = m_domain.settings().dt;
     Field *o[3] = {&out_x, &out_y, &out_z};
     const Field *s[3] = {&S_x, &S_y, &S_z};
+    double *out[3];
+    int types[3], n = 0;
     for (int a = 0; a < 3; a++) {
         bool on = false;
         for (int d : m_dir) on = on || d == a;
         if (!on) continue;
         k::add_source(m_domain.stream(), m_domain.level(0), o[a]->data, s[a]->data, dt);
-        m_domain.apply_boundary(o[a]->data, o[a]->get_type(), 0);
+        out[n] = o[a]->data;
+        types[n++] = o[a]->get_type();
     }
+    m_domain.apply_boundaries(out, types, n, 0);
     maybe_sync(m_domain, sync);
 }
 

@@ -224,7 +224,7 @@ __device__ inline void bc_item(const LevelDesc &L, const BCView &V, long long t,
         if (t < V.n_ghosts) {
             if (!ghost_coords(L, t, i, j, k)) return;
             const long long s = ghost_source(L, V.bc, i, j, k);
-            if (written(V, s)) return;  // produced by a dependent item
+            if (V.n_faces != 0 && written(V, s)) return;  // produced by a dependent item
             dst[i + static_cast<long long>(L.N[0]) * (j + static_cast<long long>(L.N[1]) * k)] =
                 ghost_chain<T>(L, V.bc, i, j, k, val(s));
             return;

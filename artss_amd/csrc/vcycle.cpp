@@ -29,7 +29,10 @@ VCycleMG::VCycleMG(Domain &d, const MultigridSettings &s) : IPressure(d), m_s(s)
         m_err1[l + 1] = std::make_unique<Field>(d, P, 0.0, l + 1);
         m_tmp[l + 1] = std::make_unique<Field>(d, P, 0.0, l + 1);
     }
-    if (d.device() >= 0) build_tail();
+    if (d.device() >= 0) {
+        d.build_mg_fills();
+        build_tail();
+    }
 }
 
 VCycleMG::~VCycleMG() {
