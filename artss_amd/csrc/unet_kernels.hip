@@ -21,7 +21,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <algorithm>
 #include <stdexcept>
+#include <type_traits>
 
 #include "unet_kernels.h"
 
@@ -54,6 +56,42 @@ __device__ inline void tap_offset(int t, int &dx, int &dy, int &dz) {
     dz = t / 9 - 1;
     dy = (t / 3) % 3 - 1;
     dx = t % 3 - 1;
+}
+
+// The four channels a lane holds of an output voxel, at element o of the
+// output: bias, activation and skip as one 8-byte write (pre: also before
+// the activation), or with GRAD the FP32 sums, zero where the BF16 activation
+// `skip` (optional) is not positive
+template <bool GRAD>
+__device__ __forceinline__ void store_tile(const f32x4 &acc, const float *bias, long long o, uint16_t *__restrict__ out,
+                                           uint16_t *__restrict__ pre, const uint16_t *__restrict__ skip, int relu,
+                                           float *__restrict__ gin) {
+    if (GRAD) {
+        float4 g{acc[0], acc[1], acc[2], acc[3]};
+        if (skip) {
+            const uint2 m = *reinterpret_cast<const uint2 *>(skip + o);
+            g.x = positive(m.x & 0xFFFFu) ? g.x : 0.f;
+            g.y = positive(m.x >> 16) ? g.y : 0.f;
+            g.z = positive(m.y & 0xFFFFu) ? g.z : 0.f;
+            g.w = positive(m.y >> 16) ? g.w : 0.f;
+        }
+        *reinterpret_cast<float4 *>(gin + o) = g;
+        return;
+    }
+    float c4[4], r[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) c4[e] = acc[e] + bias[e];
+    if (pre) *reinterpret_cast<uint2 *>(pre + o) = uint2{pack2(c4[0], c4[1]), pack2(c4[2], c4[3])};
+#pragma unroll
+    for (int e = 0; e < 4; e++) r[e] = relu ? fmaxf(c4[e], 0.f) : c4[e];
+    if (skip) {
+        const uint2 sk = *reinterpret_cast<const uint2 *>(skip + o);
+        r[0] += bf2f(static_cast<uint16_t>(sk.x & 0xFFFFu));
+        r[1] += bf2f(static_cast<uint16_t>(sk.x >> 16));
+        r[2] += bf2f(static_cast<uint16_t>(sk.y & 0xFFFFu));
+        r[3] += bf2f(static_cast<uint16_t>(sk.y >> 16));
+    }
+    *reinterpret_cast<uint2 *>(out + o) = uint2{pack2(r[0], r[1]), pack2(r[2], r[3])};
 }
 
 // ---------------------------------------------------------------- forward
@@ -194,83 +232,250 @@ __global__ void __launch_bounds__(256) k_conv_fwd(Dims D, const uint16_t *__rest
 #pragma unroll
         for (int ct = 0; ct < MT; ct++) {
             const int co = ct * 16 + 4 * kg;
-            if (GRAD) {
-                float4 g{acc[ct][j][0], acc[ct][j][1], acc[ct][j][2], acc[ct][j][3]};
-                if (skip) {
-                    const uint2 m = *reinterpret_cast<const uint2 *>(skip + v * COUT + co);
-                    g.x = positive(m.x & 0xFFFFu) ? g.x : 0.f;
-                    g.y = positive(m.x >> 16) ? g.y : 0.f;
-                    g.z = positive(m.y & 0xFFFFu) ? g.z : 0.f;
-                    g.w = positive(m.y >> 16) ? g.w : 0.f;
-                }
-                *reinterpret_cast<float4 *>(gin + v * COUT + co) = g;
-                continue;
-            }
-            float c4[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) c4[e] = acc[ct][j][e] + bias[co + e];
-            if (pre) {
-                uint2 pk;
-                pk.x = static_cast<unsigned>(f2bf(c4[0])) | (static_cast<unsigned>(f2bf(c4[1])) << 16);
-                pk.y = static_cast<unsigned>(f2bf(c4[2])) | (static_cast<unsigned>(f2bf(c4[3])) << 16);
-                *reinterpret_cast<uint2 *>(pre + v * COUT + co) = pk;
-            }
-            float r[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) r[e] = relu ? fmaxf(c4[e], 0.f) : c4[e];
-            if (skip) {
-                const uint2 sk = *reinterpret_cast<const uint2 *>(skip + v * COUT + co);
-                r[0] += bf2f(static_cast<uint16_t>(sk.x & 0xFFFFu));
-                r[1] += bf2f(static_cast<uint16_t>(sk.x >> 16));
-                r[2] += bf2f(static_cast<uint16_t>(sk.y & 0xFFFFu));
-                r[3] += bf2f(static_cast<uint16_t>(sk.y >> 16));
-            }
-            uint2 o;
-            o.x = static_cast<unsigned>(f2bf(r[0])) | (static_cast<unsigned>(f2bf(r[1])) << 16);
-            o.y = static_cast<unsigned>(f2bf(r[2])) | (static_cast<unsigned>(f2bf(r[3])) << 16);
-            *reinterpret_cast<uint2 *>(out + v * COUT + co) = o;
+            store_tile<GRAD>(acc[ct][j], bias + co, v * COUT + co, out, pre, skip, relu, gin);
         }
     }
 }
 
-// First layer: x is FP32 with CI (2) channels, 16 BF16 outputs with ReLU.
-// One voxel per thread; the 27 taps are unrolled with zero operands outside
-// the volume, so their loads are in flight together, and the 16 outputs
-// leave as two 16-byte stores.
-template <int CI, int CO>
-__global__ void k_conv_in(Dims D, const float *__restrict__ x, const float *__restrict__ W,
-                          const float *__restrict__ bias, uint16_t *__restrict__ out) {
-    static_assert(CI == 2 && CO == 16, "two input channels, sixteen outputs");
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y, z = blockIdx.z;
-    if (i >= D.X) return;
-    float2 xv[27];
+// ---- the two 16-channel layers at full resolution
+// With 16 output channels every 16-byte load of k_conv_fwd feeds one matrix
+// instruction, and each input row is loaded for all 27 taps: at 256x128x128
+// these layers were bound by the L1 (64 bytes per clock and CU: 165 and 199
+// us), three times over what memory needs.  Both kernels march along z with
+// the sums of the output planes an input plane reaches in registers, so a
+// row is loaded once per shift along x and wavefront.  A row is read through
+// a buffer descriptor of its own: voxels beyond its ends read as zero.
+__device__ __forceinline__ bf16x8 row_load(__amdgpu_buffer_rsrc_t r, unsigned offset) {
+    return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, offset, 0, 0));
+}
+// row (y, z) of a volume of C channels (outside the volume: empty)
+template <int C>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const Dims &D, const uint16_t *in, int y, int z) {
+    const bool ok = y >= 0 && y < D.Y && z >= 0 && z < D.Z;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(in + (ok ? vox(D, 0, y, z) * C : 0)),
+                                             static_cast<short>(0), ok ? D.X * 2 * C : 0, 0x00020000);
+}
+constexpr unsigned kNowhere = 0x80000000u;  // an offset beyond any row
+
+// 16 -> 16 channels at one resolution (k_conv_fwd's arguments).  A wavefront
+// owns 16 voxels along x and kRows16 rows, with the weights of all taps in
+// registers: per row of taps one operand for the voxels x - 1 and x, one for
+// x + 1 (its other half zero).  At 256x128x128 165 -> 88 us (57 to read and
+// write the volume once), its gradient form at 128x64x64 30 -> 21 us; loading
+// the next plane ahead takes the second wavefront per SIMD (130 us).
+constexpr int kRows16 = 4;
+template <bool GRAD>
+__global__ void __launch_bounds__(256) k_conv16(Dims D, const uint16_t *__restrict__ in, const uint16_t *__restrict__ Wt,
+                                                const float *__restrict__ bias, uint16_t *__restrict__ out,
+                                                uint16_t *__restrict__ pre, const uint16_t *__restrict__ skip, int relu,
+                                                float *__restrict__ gin, int planes) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int col = lane & 15, kg = lane >> 4;
+    const int x0 = static_cast<int>(blockIdx.x) * 16, y0 = (static_cast<int>(blockIdx.y) * 4 + wave) * kRows16;
+    const int z0 = static_cast<int>(blockIdx.z) * planes, z1 = min(z0 + planes, D.Z);
+    if (y0 >= D.Y) return;  // no workgroup barrier in this kernel
+    const bf16x8 zero8 = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
+    bf16x8 a[9][2];  // [3 (dz + 1) + dy + 1 of the input row][voxels x - 1 and x; x + 1]
 #pragma unroll
-    for (int t = 0; t < 27; t++) {
-        int dx, dy, dz;
-        tap_offset(t, dx, dy, dz);
-        const int xx = i + dx, yy = y + dy, zz = z + dz;
-        const bool inside = xx >= 0 && xx < D.X && yy >= 0 && yy < D.Y && zz >= 0 && zz < D.Z;
-        xv[t] = inside ? *reinterpret_cast<const float2 *>(x + vox(D, xx, yy, zz) * CI) : make_float2(0.f, 0.f);
-    }
-    float acc[CO];
+    for (int r = 0; r < 9; r++)
 #pragma unroll
-    for (int c = 0; c < CO; c++) acc[c] = bias[c];
-#pragma unroll
-    for (int t = 0; t < 27; t++)
-#pragma unroll
-        for (int c = 0; c < CO; c++) {
-            acc[c] += xv[t].x * W[(t * CI + 0) * CO + c];
-            acc[c] += xv[t].y * W[(t * CI + 1) * CO + c];
+        for (int q = 0; q < 2; q++) {
+            const int d = q == 0 ? kg >> 1 : 2;
+            const int t = GRAD ? (8 - r) * 3 + 2 - d : r * 3 + d;
+            const bf16x8 w =
+                __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(Wt + (t * 16 + col) * 16 + 8 * (kg & 1)));
+            a[r][q] = q == 1 && kg >= 2 ? zero8 : w;
         }
-    unsigned pk[CO / 2];
+    const int left = (x0 + col - 1) * 32 + 16 * kg;
+    const unsigned off0 = left < 0 ? kNowhere : static_cast<unsigned>(left);
+    const unsigned off1 = kg >= 2 ? kNowhere : static_cast<unsigned>((x0 + col + 1) * 32 + 16 * kg);
+    f32x4 acc[3][kRows16];
+    // input plane z0 - 1 + q, q % 3 == PH: starts output plane z0 + q (slot
+    // PH), ends z0 + q - 2 (slot PH + 1 mod 3)
+    auto plane = [&](auto ph, int q) {
+        constexpr int PH = decltype(ph)::value;
+        const int zi = z0 - 1 + q;
 #pragma unroll
-    for (int c = 0; c < CO; c += 2)
-        pk[c / 2] = static_cast<unsigned>(f2bf(fmaxf(acc[c], 0.f))) |
-                    (static_cast<unsigned>(f2bf(fmaxf(acc[c + 1], 0.f))) << 16);
-    uint4 *o = reinterpret_cast<uint4 *>(out + vox(D, i, y, z) * CO);
-    o[0] = uint4{pk[0], pk[1], pk[2], pk[3]};
-    o[1] = uint4{pk[4], pk[5], pk[6], pk[7]};
+        for (int o = 0; o < kRows16; o++) acc[PH][o] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (zi >= 0 && zi < D.Z) {
+            bf16x8 b[kRows16 + 2][2];
+#pragma unroll
+            for (int r = 0; r < kRows16 + 2; r++) {
+                const auto buf = row_buffer<16>(D, in, y0 - 1 + r, zi);
+                b[r][0] = row_load(buf, off0);
+                b[r][1] = row_load(buf, off1);
+            }
+#pragma unroll
+            for (int r = 0; r < kRows16 + 2; r++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int dz = 0; dz < 3; dz++)
+#pragma unroll
+                        for (int dy = 0; dy < 3; dy++) {
+                            const int o = r - dy;
+                            if (o < 0 || o >= kRows16) continue;
+                            f32x4 &c = acc[(PH + 3 - dz) % 3][o];
+                            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[3 * dz + dy][h], b[r][h], c, 0, 0, 0);
+                        }
+        }
+        const int z = zi - 1;
+        if (z < z0 || z >= z1 || x0 + col >= D.X) return;
+#pragma unroll
+        for (int o = 0; o < kRows16; o++)
+            if (y0 + o < D.Y)
+                store_tile<GRAD>(acc[(PH + 1) % 3][o], bias + 4 * kg, vox(D, x0 + col, y0 + o, z) * 16 + 4 * kg, out, pre,
+                                 skip, relu, gin);
+    };
+#pragma unroll 1
+    for (int q = 0; q < z1 - z0 + 2; q += 3) {
+        plane(std::integral_constant<int, 0>(), q);
+        if (q + 1 < z1 - z0 + 2) plane(std::integral_constant<int, 1>(), q + 1);
+        if (q + 2 < z1 - z0 + 2) plane(std::integral_constant<int, 2>(), q + 2);
+    }
+}
+
+// 32 -> 16 channels, the input upsampled (k_conv_fwd's UP form).  A wavefront
+// owns 16 coarse voxels along x and two coarse rows, that is 2 x 2 parities
+// of four fine rows, and marches through the coarse planes: plane c ends the
+// fine planes 2 c - 1 and 2 c and starts 2 c + 1 and 2 c + 2.  The 64 weight
+// operands lie in LDS, each read once per plane for two rows.  At 256x128x128
+// 199 -> 170 us, with two wavefronts per SIMD to hide the loads (64 us of
+// memory); the next plane ahead needs more registers than two leave (259 us).
+__global__ void __launch_bounds__(256) k_conv_up16(Dims D, const uint16_t *__restrict__ in,
+                                                   const uint16_t *__restrict__ Wt, const float *__restrict__ bias,
+                                                   uint16_t *__restrict__ out, uint16_t *__restrict__ pre,
+                                                   const uint16_t *__restrict__ skip, int relu, int planes) {
+    __shared__ uint4 weights[64][64];  // [parity][tap], as a lane reads it
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int col = lane & 15, kg = lane >> 4;
+    const Dims C{D.X >> 1, D.Y >> 1, D.Z >> 1};
+    for (int m = wave; m < 64; m += 4)
+        weights[m][lane] = *reinterpret_cast<const uint4 *>(Wt + (m * 16 + col) * 32 + 8 * kg);
+    __syncthreads();
+    const int x0 = static_cast<int>(blockIdx.x) * 16, y0 = (static_cast<int>(blockIdx.y) * 4 + wave) * 2;
+    const int c0 = static_cast<int>(blockIdx.z) * planes, c1 = min(c0 + planes, C.Z);
+    if (y0 >= C.Y) return;  // no workgroup barrier from here on
+    unsigned off[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const int o = (x0 + col - 1 + d) * 64 + 16 * kg;
+        off[d] = o < 0 ? kNowhere : static_cast<unsigned>(o);
+    }
+    f32x4 acc[2][2][2][2][2];  // [pair of fine planes, by parity of c][odd plane first][coarse row][y parity][x parity]
+    auto plane = [&](auto ph, int c) {
+        constexpr int END = decltype(ph)::value, BEGIN = 1 - END;
+#pragma unroll
+        for (int n = 0; n < 16; n++)
+            acc[BEGIN][n >> 3][(n >> 2) & 1][(n >> 1) & 1][n & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (c >= 0 && c < C.Z) {
+            bf16x8 b[4][3];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const auto buf = row_buffer<32>(C, in, y0 - 1 + r, c);
+#pragma unroll
+                for (int d = 0; d < 3; d++) b[r][d] = row_load(buf, off[d]);
+            }
+#pragma unroll
+            for (int m = 0; m < 64; m++) {
+                const int px = (m >> 3) & 1, py = (m >> 4) & 1, pz = m >> 5, ox = m & 1, oy = (m >> 1) & 1, oz = (m >> 2) & 1;
+                const bf16x8 w = __builtin_bit_cast(bf16x8, weights[m][lane]);
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    f32x4 &s = acc[oz == 1 ? END : BEGIN][1 - pz][r][py][px];
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, b[r + py + oy][px + ox], s, 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < 16; n++) {
+            const int even = n >> 3, r = (n >> 2) & 1, py = (n >> 1) & 1, px = n & 1;
+            const int z = 2 * c - 1 + even, y = 2 * (y0 + r) + py, x = 2 * (x0 + col) + px;
+            if (z >= 2 * c0 && z < 2 * c1 && y < D.Y && x < D.X)
+                store_tile<false>(acc[END][even][r][py][px], bias + 4 * kg, vox(D, x, y, z) * 16 + 4 * kg, out, pre, skip,
+                                  relu, nullptr);
+        }
+    };
+#pragma unroll
+    for (int n = 0; n < 16; n++) acc[0][n >> 3][(n >> 2) & 1][(n >> 1) & 1][n & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int c = c0 - 1; c <= c1; c += 2) {
+        plane(std::integral_constant<int, 0>(), c);
+        if (c + 1 <= c1) plane(std::integral_constant<int, 1>(), c + 1);
+    }
+}
+
+// First layer: two FP32 channels to 16 BF16 with ReLU, on
+// v_mfma_f32_16x16x4_f32 (FP32 operands and sums) in the manner of k_conv16:
+// a K step is two voxels of two channels.  A row of three taps is one step
+// for the voxels x - 1 and x; the voxels x + 1 of two rows share one, so a
+// plane of taps is five steps.  One thread per voxel with 864 multiply-adds was
+// bound by their issue: 169 us at 256x128x128, 106 now (58 of matrix issue).
+__global__ void __launch_bounds__(256) k_conv_in(Dims D, const float *__restrict__ x, const float *__restrict__ W,
+                                                 const float *__restrict__ bias, uint16_t *__restrict__ out,
+                                                 int planes) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int col = lane & 15, kg = lane >> 4;
+    const int x0 = static_cast<int>(blockIdx.x) * 16, y0 = (static_cast<int>(blockIdx.y) * 4 + wave) * kRows16;
+    const int z0 = static_cast<int>(blockIdx.z) * planes, z1 = min(z0 + planes, D.Z);
+    if (y0 >= D.Y) return;  // no workgroup barrier in this kernel
+    auto weight = [&](int t, int ci) { return W[(t * 2 + ci) * 16 + col]; };
+    float a[3][5];  // [dz + 1][rows dy = -1, 0, 1 at x - 1 and x; x + 1 of rows -1 and 0; x + 1 of row 1]
+#pragma unroll
+    for (int dz = 0; dz < 3; dz++) {
+#pragma unroll
+        for (int dy = 0; dy < 3; dy++) a[dz][dy] = weight((dz * 3 + dy) * 3 + (kg >> 1), kg & 1);
+        a[dz][3] = weight((dz * 3 + (kg >> 1)) * 3 + 2, kg & 1);
+        a[dz][4] = kg < 2 ? weight((dz * 3 + 2) * 3 + 2, kg & 1) : 0.f;
+    }
+    const int left = (x0 + col - 1) * 8 + 4 * kg;
+    const unsigned off0 = left < 0 ? kNowhere : static_cast<unsigned>(left);
+    const unsigned right = static_cast<unsigned>((x0 + col + 1) * 8 + 4 * (kg & 1));
+    const unsigned off_lo = kg < 2 ? right : kNowhere, off_hi = kg < 2 ? kNowhere : right;
+    f32x4 acc[3][kRows16];
+    auto plane = [&](auto ph, int q) {
+        constexpr int PH = decltype(ph)::value;
+        const int zi = z0 - 1 + q;
+#pragma unroll
+        for (int o = 0; o < kRows16; o++) acc[PH][o] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (zi >= 0 && zi < D.Z) {
+            unsigned b0[kRows16 + 2], lo[kRows16 + 2], hi[kRows16 + 2];
+#pragma unroll
+            for (int r = 0; r < kRows16 + 2; r++) {
+                const int y = y0 - 1 + r;
+                const bool ok = y >= 0 && y < D.Y;
+                const auto buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(x + (ok ? vox(D, 0, y, zi) * 2 : 0)),
+                                                                   static_cast<short>(0), ok ? D.X * 8 : 0, 0x00020000);
+                b0[r] = __builtin_amdgcn_raw_buffer_load_b32(buf, off0, 0, 0);
+                lo[r] = __builtin_amdgcn_raw_buffer_load_b32(buf, off_lo, 0, 0);
+                hi[r] = r >= 1 && r <= kRows16 ? __builtin_amdgcn_raw_buffer_load_b32(buf, off_hi, 0, 0) : 0u;
+            }
+#pragma unroll
+            for (int o = 0; o < kRows16; o++)
+#pragma unroll
+                for (int dz = 0; dz < 3; dz++) {
+                    f32x4 &c = acc[(PH + 3 - dz) % 3][o];
+#pragma unroll
+                    for (int dy = 0; dy < 3; dy++)
+                        c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[dz][dy], __uint_as_float(b0[o + dy]), c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[dz][3], __uint_as_float(lo[o] | hi[o + 1]), c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[dz][4], __uint_as_float(lo[o + 2]), c, 0, 0, 0);
+                }
+        }
+        const int z = zi - 1;
+        if (z < z0 || z >= z1 || x0 + col >= D.X) return;
+#pragma unroll
+        for (int o = 0; o < kRows16; o++)
+            if (y0 + o < D.Y)
+                store_tile<false>(acc[(PH + 1) % 3][o], bias + 4 * kg, vox(D, x0 + col, y0 + o, z) * 16 + 4 * kg, out,
+                                  nullptr, nullptr, 1, nullptr);
+    };
+#pragma unroll 1
+    for (int q = 0; q < z1 - z0 + 2; q += 3) {
+        plane(std::integral_constant<int, 0>(), q);
+        if (q + 1 < z1 - z0 + 2) plane(std::integral_constant<int, 1>(), q + 1);
+        if (q + 2 < z1 - z0 + 2) plane(std::integral_constant<int, 2>(), q + 2);
+    }
 }
 
 // Last layer: CI BF16 channels -> one FP32 output, no activation.  A thread
@@ -313,9 +518,9 @@ __global__ void k_conv_out(Dims D, const uint16_t *__restrict__ in, const float 
                     for (int e = 0; e < 8; e++) {
                         const float v = bf2f(static_cast<uint16_t>((w4[e >> 1] >> (16 * (e & 1))) & 0xFFFFu));
                         const int ci = 8 * g + e;
-                        if (r < NZ) acc[r] += v * W[tb * CI + ci];
-                        if (r >= 1 && r - 1 < NZ) acc[r - 1] += v * W[(9 + tb) * CI + ci];
-                        if (r >= 2) acc[r - 2] += v * W[(18 + tb) * CI + ci];
+                        if (r < NZ) acc[r] = fmaf(v, W[tb * CI + ci], acc[r]);
+                        if (r >= 1 && r - 1 < NZ) acc[r - 1] = fmaf(v, W[(9 + tb) * CI + ci], acc[r - 1]);
+                        if (r >= 2) acc[r - 2] = fmaf(v, W[(18 + tb) * CI + ci], acc[r - 2]);
                     }
                 }
             }
@@ -959,12 +1164,44 @@ inline unsigned blocks_for(long long n) {
 }  // namespace
 
 // ---------------------------------------------------------------- launchers
-#define ARTSS_CONV_CASES(X) X(16, 16) X(16, 32) X(32, 64) X(64, 64) X(64, 32) X(32, 16)
+#define ARTSS_CONV_CASES(X) X(16, 32) X(32, 64) X(64, 64) X(64, 32) X(32, 16)
 // voxels per wavefront row of k_conv_fwd: 16 x NV, eight matrix tiles per K step
 constexpr int row_tiles(int co) { return co == 16 ? 8 : (co == 32 ? 4 : 2); }
 
+// Planes per wavefront of the marching kernels, for `columns` wavefronts per
+// plane of `z`: four wavefronts per SIMD if the volume has them, within 4
+// planes (half the planes read are then halo) and 16
+int march_planes(long long columns, int z) {
+    const long long p = z * columns / 4096;
+    return static_cast<int>(std::min(16LL, std::max(4LL, p)));
+}
+template <bool GRAD>
+void launch_conv16(hipStream_t s, Dims D, const uint16_t *in, const uint16_t *Wt, const float *bias, uint16_t *out,
+                   uint16_t *pre, const uint16_t *skip, bool relu, float *gin) {
+    const int gx = (D.X + 15) / 16, gy = (D.Y + 4 * kRows16 - 1) / (4 * kRows16);
+    const int planes = march_planes(4LL * gx * gy, D.Z);
+    k_conv16<GRAD><<<dim3(gx, gy, (D.Z + planes - 1) / planes), 256, 0, s>>>(D, in, Wt, bias, out, pre, skip, relu ? 1 : 0,
+                                                                            gin, planes);
+}
+
 void conv_fwd(hipStream_t s, int cin, int cout, bool up, Dims D, const uint16_t *in, const uint16_t *Wt,
               const float *bias, uint16_t *out, uint16_t *pre, const uint16_t *skip, bool relu) {
+    if (cin == 16 && cout == 16 && !up) {
+        launch_conv16<false>(s, D, in, Wt, bias, out, pre, skip, relu, nullptr);
+        return;
+    }
+    if (cin == 32 && cout == 16 && up) {
+        const int cx = D.X >> 1, cy = D.Y >> 1, cz = D.Z >> 1;
+        const int gx = (cx + 15) / 16, gy = (cy + 7) / 8, planes = march_planes(4LL * gx * gy, cz);
+        const int gz = (cz + planes - 1) / planes;
+        // two workgroups of its 64 KiB fit a CU: it needs about that many to
+        // beat k_conv_fwd (256x128x128, 1024 workgroups: 170 against 199 us;
+        // 128x64x64, 128 workgroups: 59 against 32 us)
+        if (gx * gy * gz >= 512) {
+            k_conv_up16<<<dim3(gx, gy, gz), 256, 0, s>>>(D, in, Wt, bias, out, pre, skip, relu ? 1 : 0, planes);
+            return;
+        }
+    }
 #define CASE(CI, CO)                                                                                             \
     if (cin == CI && cout == CO) {                                                                              \
         constexpr int NV = row_tiles(CO);                                                                       \
@@ -988,6 +1225,10 @@ void conv_fwd(hipStream_t s, int cin, int cout, bool up, Dims D, const uint16_t 
 
 void conv_dgrad(hipStream_t s, int cin, int cout, Dims D, const uint16_t *g, const uint16_t *W, const uint16_t *act,
                 float *gin) {
+    if (cin == 16 && cout == 16) {
+        launch_conv16<true>(s, D, g, W, nullptr, nullptr, nullptr, act, false, gin);
+        return;
+    }
 #define CASE(CI, CO)                                                                                             \
     if (cin == CI && cout == CO) {                                                                              \
         constexpr int NV = row_tiles(CI);                                                                       \
@@ -996,7 +1237,7 @@ void conv_dgrad(hipStream_t s, int cin, int cout, Dims D, const uint16_t *g, con
             <<<grid, 256, 0, s>>>(D, g, W, nullptr, nullptr, nullptr, act, 0, gin);                             \
         return;                                                                                                 \
     }
-    CASE(16, 16) CASE(16, 32) CASE(32, 64) CASE(64, 64)
+    CASE(16, 32) CASE(32, 64) CASE(64, 64)
 #undef CASE
     throw std::invalid_argument("conv_dgrad: unsupported channel pair");
 }
@@ -1051,7 +1292,9 @@ void conv_wgrad(hipStream_t s, int cin, int cout, bool up, Dims D, const uint16_
 }
 
 void conv_in(hipStream_t s, Dims D, const float *x, const float *W, const float *bias, uint16_t *out) {
-    k_conv_in<2, 16><<<dim3((D.X + 63) / 64, D.Y, D.Z), 64, 0, s>>>(D, x, W, bias, out);
+    const int gx = (D.X + 15) / 16, gy = (D.Y + 4 * kRows16 - 1) / (4 * kRows16);
+    const int planes = march_planes(4LL * gx * gy, D.Z);
+    k_conv_in<<<dim3(gx, gy, (D.Z + planes - 1) / planes), 256, 0, s>>>(D, x, W, bias, out, planes);
 }
 void conv_out(hipStream_t s, Dims D, const uint16_t *in, const float *W, const float *bias, float *y) {
     k_conv_out<16, 8><<<dim3((D.X + 63) / 64, (D.Y + 3) / 4, (D.Z + 7) / 8), dim3(64, 4, 1), 0, s>>>(D, in, W, bias, y);

@@ -46,3 +46,35 @@ def test_gradients_match_reference(X, Y, Z):
     again, g2 = net.gradients(xb, tb)
     assert again == loss and np.array_equal(g, g2)
     assert net.gradients(xb, tb, want_grads=False)[0] == loss
+
+
+def test_forward_of_a_large_volume_matches_its_corners():
+    """The marching kernel of the last upsampling layer serves large volumes
+    only.  An output voxel depends on inputs at most 40 voxels away (8 at the
+    coarsest level and its upsampling, 8 + 4 + 3 at the finer ones, rounded up
+    to whole coarse voxels), so the two far corners of a large volume with
+    partial tiles must repeat in 96-voxel boxes cut from it, which take the
+    small volumes' kernel.  The two sum in different orders in FP32: a BF16
+    activation may differ by one rounding (2^-8), in each of eight layers."""
+    X, Y, Z = 168, 136, 136
+    dom = artss_amd.Domain(cases.ns_taylor_green(n=16, levels=2, steps=1))
+    rng = np.random.default_rng(11)
+    net = artss_amd.UNet(dom, seed=3)
+    p = U.init_params(seed=5)
+    for n, *_ in U.LAYERS:
+        p[n + ".W"] = rng.standard_normal(p[n + ".W"].shape) * np.sqrt(2.0 / (27 * p[n + ".W"].shape[-2]))
+    net.set_params(_flat(p))
+    x = rng.standard_normal((Z, Y, X, 2)).astype(np.float32)
+
+    def forward(v):
+        out = artss_amd.Buffer(dom, np.zeros(v.shape[:3] + (1,), np.float32))
+        net.forward(artss_amd.Buffer(dom, np.ascontiguousarray(v)), out)
+        return out.download()[..., 0]
+
+    whole = forward(x)
+    assert np.isfinite(whole).all() and np.any(whole)
+    low, high = forward(x[:96, :96, :96]), forward(x[-96:, -96:, -96:])
+    for part, ref in ((low[:48, :48, :48], whole[:48, :48, :48]), (high[-48:, -48:, -48:], whole[-48:, -48:, -48:])):
+        err = float(np.linalg.norm(part - ref) / np.linalg.norm(ref))
+        print("relative difference", err)
+        assert err < np.sqrt(8) * 2.0 ** -8
