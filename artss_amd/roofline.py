@@ -72,6 +72,27 @@ class Levels:
                 return l, "full"
         return None, None
 
+    def level_of_coarse(self, gx, gy, gz):
+        """coarse level of a k_residuum_restrict launch: 64 x 4 workgroups over its inner box (or, the
+        coarsest, its whole array), one plane each"""
+        for l, (n, N) in enumerate(zip(self.n, self.N)):
+            for v in (n, N):
+                if l > 0 and gx == -(-v[0] // 64) * 64 and gy == -(-v[1] // 4) * 4 and gz == v[2]:
+                    return l
+        return None
+
+    def level_of_tiles(self, threads, fp32):
+        """level of a k_smooth_start launch: the tiles of mg_fused.hip, then the fill items (fewer
+        workgroups than tiles of the next finer level)"""
+        best = None
+        for l, n in enumerate(self.n):
+            gx = -(-n[0] // 64)
+            ty, tz = (2, 4) if gx * n[1] * n[2] < 16384 else ((6, 4) if fp32 else (2, 8))
+            tiles = gx * -(-n[1] // ty) * -(-n[2] // tz)
+            if tiles * 256 <= threads and (best is None or tiles > best[1]):
+                best = (l, tiles)
+        return best[0] if best else None
+
     def level_of_1d(self, threads):
         """whole-array element-wise launch: the level whose array fits the grid"""
         for l in range(len(self.n)):
@@ -139,12 +160,30 @@ def bytes_of(kernel, args, gx, gy, gz, L, turbulent=True, tail_cells=4096):
     if kernel in ("k_gcr_coef", "k_sum", "k_sum_gate", "k_reduce_gate", "k_reduce_sum", "k_gate_open",
                   "k_gate_open_iter"):
         return 8 * 4 * L.inner(0) // (BX * BY * 4), "partial sums (latency bound)"
+    if kernel == "k_smooth_start":
+        t, tb, tc = (size_of(a) for a in args[:3])
+        from_b, coarse = args[3] == "true", args[4] == "true"
+        l = L.level_of_tiles(gx, t == 4)
+        if l is None:
+            return None, "level unknown"
+        per = tb + t + (0 if from_b else t)
+        extra = tc * L.inner(l + 1) if coarse and l + 1 < len(L.n) else 0
+        return per * L.inner(l) + extra, "level %d: read %sb%s, write one sweep" % (
+            l, "" if from_b else "x, ", ", coarse" if coarse else "")
+    if kernel == "k_residuum_restrict":
+        l = L.level_of_coarse(gx, gy, gz)
+        if l is None:
+            return None, "level unknown"
+        t, tb, tout = (size_of(a) for a in args[:3])
+        per = tb + (0 if args[3] == "true" else t)
+        return per * L.inner(l - 1) + tout * L.inner(l), "to level %d: read %sb, write the restricted residuum" % (
+            l, "" if args[3] == "true" else "x, ")
     if kernel == "k_bc_domain":
         l = next((q for q in range(len(L.n)) if gx == -(-L.ghosts(q) // 256) * 256), None)
         if l is None:
             return None, "level unknown"
         return 16 * L.ghosts(l), "ghost cells: read source, write ghost, level %d" % l
-    if kernel in ("k_bc_faces", "k_fill_bc", "k_bc_merged"):
+    if kernel in ("k_bc_faces", "k_fill_bc", "k_fill_bcs", "k_bc_merged"):
         return 16 * gx * max(1, gy) * max(1, gz), "at most one entry per thread: read neighbour, write cell"
     if level is None:
         return None, "level unknown"
@@ -167,9 +206,6 @@ def bytes_of(kernel, args, gx, gy, gz, L, turbulent=True, tail_cells=4096):
     if kernel == "k_prolongate_add_bc":
         tf, tc = size_of(args[0]), size_of(args[1])
         return (2 * tf) * cells + tc * L.inner(level + 1), "to level %d: read fine, coarse; write" % level
-    if kernel == "k_restrict_sweep0":
-        # grid over the coarse array; 8 fine FP32 reads per coarse cell, write rhs and error
-        return (8 * 4 + 4 + 4) * cells, "to level %d: read 8 fine, write rhs and first sweep" % level
     if kernel == "k_restrict_fill":
         tin, tout = size_of(args[0]), size_of(args[1])
         terr = size_of(args[2]) if len(args) > 2 else 8
@@ -182,7 +218,7 @@ def bytes_of(kernel, args, gx, gy, gz, L, turbulent=True, tail_cells=4096):
     if kernel == "k_copy_bc":
         return 16 * (cells if kind == "inner" else whole), "copy with fill, level %d" % level
     per = {
-        "k_sl_advect": 40, "k_jacobi_diffuse": 24 + ev, "k_jacobi_mg": 24, "k_jacobi_mg_first": 24,
+        "k_sl_advect": 40, "k_sl_advect_bc": 40, "k_jacobi_diffuse": 24 + ev, "k_jacobi_iter": 24 + ev, "k_jacobi_mg": 24, "k_jacobi_mg_first": 24,
         "k_explicit_diffuse": 16 + ev, "k_dissipate": 40, "k_update_norm": 16 + ev, "k_residuum": 24,
         "k_residual_partials": 16, "k_residual_vec": 24, "k_divergence": 32, "k_projection": 56,
         "k_smagorinsky": 32, "k_add_source": 24, "k_buoyancy": 24, "k_copy_domain": 16, "k_warm_partials": 16,
