@@ -224,7 +224,15 @@ __device__ inline void bc_item(const LevelDesc &L, const BCView &V, long long t,
         if (t < V.n_ghosts) {
             if (!ghost_coords(L, t, i, j, k)) return;
             const long long s = ghost_source(L, V.bc, i, j, k);
-            if (V.n_faces != 0 && written(V, s)) return;  // produced by a dependent item
+            // produced by a dependent item (obstacle faces lie in the boxes: the bitmap is only read there, which
+            // spares the first fill of a field 0.1 MB of untranslated pages per million cells)
+            if (V.n_faces != 0) {
+                const unsigned u = static_cast<unsigned>(s), Nx = static_cast<unsigned>(L.N[0]), Ny = static_cast<unsigned>(L.N[1]);
+                if (in_obstacle(L, static_cast<int>(u % Nx), static_cast<int>((u / Nx) % Ny),
+                                static_cast<int>(u / (Nx * Ny))) &&
+                    written(V, s))
+                    return;
+            }
             dst[i + static_cast<long long>(L.N[0]) * (j + static_cast<long long>(L.N[1]) * k)] =
                 ghost_chain<T>(L, V.bc, i, j, k, val(s));
             return;
